@@ -471,7 +471,7 @@ int64_t replay_trace_f32(const void *packet, int32_t nx, int32_t ny, int32_t nz,
       double *o = trace + 12 * k;
       o[0] = t.u0; o[1] = t.u1; o[2] = t.u2;
       o[3] = t.o0; o[4] = t.o1; o[5] = t.o2;
-      o[6] = t.s; o[7] = t.w; o[8] = t.cell; o[9] = t.ijk; o[10] = t.ctr; o[11] = t.outcome;
+      o[6] = t.s; o[7] = t.w * fpm::pow2d(kc.eq); o[8] = t.cell; o[9] = t.ijk; o[10] = t.ctr; o[11] = t.outcome;
       ++k;
     }
     return k;

@@ -52,6 +52,15 @@ STORM_HD double quantize_unbiased(double v, int e, uint32_t u24) {
   return (u < frac ? fl + 1.0 : fl) * fpm::pow2d(e);
 }
 
+// Draw of carry_round, 24 bits.
+STORM_HD uint32_t carry_draw(uint32_t id, uint32_t ctr, uint32_t cell) {
+  uint32_t h = id * 0x2545F491u ^ (ctr + 0x3C6EF372u) * 0x9E3779B9u ^ cell * 0x27D4EB2Fu;
+  h ^= h >> 16;
+  h *= 0x7FEB352Du;
+  h ^= h >> 15;
+  return h >> 8;
+}
+
 // The weight a packet carries on after a cell visit (into the next cell, to
 // census or out of the problem), as a multiple of 2^e: w rounded without
 // bias, the draw a hash of the packet id, its random-stream position and the
@@ -60,11 +69,7 @@ STORM_HD double quantize_unbiased(double v, int e, uint32_t u24) {
 // take up to one quantum from a packet at each face it crosses, which ends
 // packets of a few quanta long before their physics does.
 STORM_HD double carry_round(double w, double w_enter, int e, uint32_t id, uint32_t ctr, uint32_t cell) {
-  uint32_t h = id * 0x2545F491u ^ (ctr + 0x3C6EF372u) * 0x9E3779B9u ^ cell * 0x27D4EB2Fu;
-  h ^= h >> 16;
-  h *= 0x7FEB352Du;
-  h ^= h >> 15;
-  const double wq = quantize_unbiased(w, e, h >> 8);
+  const double wq = quantize_unbiased(w, e, carry_draw(id, ctr, cell));
   return wq > w_enter ? quantize_down(w, e) : wq;
 }
 
@@ -80,6 +85,35 @@ STORM_HD double emission_round(double per, int e, uint32_t cell, uint32_t step) 
   h ^= h >> 15;
   return quantize_unbiased(per, e, h >> 8);
 }
+
+// The integer below 2^63 that the integral double y holds (5 instructions: a
+// double to 64-bit integer conversion also truncates).
+STORM_HD uint64_t to_u64(double y) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const double hi = __builtin_floor(y * 0x1p-32);
+  const double lo = __builtin_fma(hi, -0x1p32, y);
+  return (static_cast<uint64_t>(static_cast<uint32_t>(hi)) << 32) | static_cast<uint32_t>(lo);
+#else
+  return static_cast<uint64_t>(y);
+#endif
+}
+
+// carry_round on weights in quanta: w (in quanta) rounded without bias to an
+// integer no larger than n_enter, the visit's beginning weight; `w` becomes
+// that integer as a double, which the return value is too.  The same numbers
+// as carry_round gives on w 2^e.
+STORM_HD uint64_t carry_round_q(double &w, uint64_t n_enter, uint32_t draw) {
+  const double fl = floor(w);
+  const double u = static_cast<double>(draw) * 0x1p-24;
+  uint64_t n = to_u64(fl);
+  const bool up = u < w - fl && n < n_enter;
+  w = up ? fl + 1.0 : fl;
+  n += up ? 1u : 0u;
+  return n;
+}
+
+// An integer below 2^62 as limbs.
+STORM_HD Limbs limbs_of_value(uint64_t v) { return Limbs{v & kLoMask, v >> kLoBits}; }
 
 // Limbs of w / 2^e for a w that is an integer multiple of 2^e below 2^62.
 STORM_HD Limbs limbs_of(double w, int e) {

@@ -18,6 +18,10 @@
 //   expm1 : Taylor series to y^9 for |y| < ln2/2, exp(y) - 1 otherwise.
 //   sincos of 2*pi*u : exact quadrant reduction of 4u, Taylor series of sin
 //           and cos on [-pi/4, pi/4].
+//   1/x, sqrt, a/b (recip_f, sqrt_f, div_f): the hardware's 1 ulp estimate
+//           and one Newton step with a fused remainder, which rounds as IEEE
+//           does over the ranges stated at each (checked for every float of
+//           the range on gfx950); the host uses the IEEE operators.
 // Accuracy is a few ulp, far below Monte Carlo noise; what matters is that
 // host and device produce the same bits.
 #pragma once
@@ -60,6 +64,43 @@ STORM_HD float fma_f(float a, float b, float c) {
 #endif
 }
 
+// 1 / x as IEEE rounds it, for 2^-126 <= |x| <= 2^126 (3 instructions; the
+// compiler's full-range division takes 10).
+STORM_HD float recip_f(float x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const float r = __builtin_amdgcn_rcpf(x);
+  return __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r);
+#else
+  return 1.0f / x;
+#endif
+}
+
+// sqrt(x) as IEEE rounds it, for 2^-100 <= x <= 2^100 and for 0.
+STORM_HD float sqrt_f(float x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const float y = __builtin_amdgcn_rsqf(x);
+  const float g = x * y;
+  const float q = __builtin_fmaf(__builtin_fmaf(-g, g, x), 0.5f * y, g);
+  return x > 0.0f ? q : 0.0f;
+#else
+  return ::sqrtf(x);
+#endif
+}
+
+// a / b as IEEE rounds it, for b within [2^-60, 2^60] and a 0 or within
+// [2^-60, 2^60] (signs free): with the correctly rounded reciprocal the
+// quotient corrected by its exact remainder is correctly rounded (Markstein
+// 1990).
+STORM_HD float div_f(float a, float b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const float y = recip_f(b);
+  const float q = a * y;
+  return __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+#else
+  return a / b;
+#endif
+}
+
 constexpr float kLn2Hi = 0.693115234375f;          // 12 significant bits
 constexpr float kLn2Lo = 3.194618329871446e-05f;   // ln2 - kLn2Hi
 constexpr float kLog2e = 1.4426950216293335f;
@@ -92,6 +133,37 @@ STORM_HD float logf_d(float x) {
   p = fma_f(z, p, 1.0f);
   float lm = 2.0f * s * p;
   float ef = static_cast<float>(e);
+  return fma_f(ef, kLn2Hi, fma_f(ef, kLn2Lo, lm));
+}
+
+// logf_d for the uniforms: the same bits for normal x in (0, 1], without the
+// cases logf_d tells apart first (0, negative, NaN and subnormal arguments;
+// some finite value for 0).  The quotient (m - 1) / (m + 1) needs no reciprocal
+// step: the corrected estimate is the IEEE quotient for every m.
+STORM_HD float log_unit(float x) {
+  const uint32_t b = f2u(x);
+  int e = static_cast<int>(b >> 23) - 127;
+  float m = u2f((b & 0x007fffffu) | 0x3f800000u);  // [1, 2)
+  const bool up = m > kSqrt2;
+  m = up ? m * 0.5f : m;
+  e = up ? e + 1 : e;
+  const float f = m - 1.0f;
+#if defined(__HIP_DEVICE_COMPILE__)
+  const float d = 2.0f + f;
+  const float y = __builtin_amdgcn_rcpf(d);
+  const float q = f * y;
+  const float s = __builtin_fmaf(__builtin_fmaf(-d, q, f), y, q);
+#else
+  const float s = f / (2.0f + f);
+#endif
+  const float z = s * s;
+  float p = 1.0f / 9.0f;
+  p = fma_f(z, p, 1.0f / 7.0f);
+  p = fma_f(z, p, 1.0f / 5.0f);
+  p = fma_f(z, p, 1.0f / 3.0f);
+  p = fma_f(z, p, 1.0f);
+  const float lm = 2.0f * s * p;
+  const float ef = static_cast<float>(e);
   return fma_f(ef, kLn2Hi, fma_f(ef, kLn2Lo, lm));
 }
 
@@ -135,6 +207,31 @@ STORM_HD float expm1f_d(float y) {
     return fma_f(y * y, p, y);
   }
   return expf_d(y) - 1.0f;
+}
+
+// expm1f_d for y <= 0, the same bits in one straight line: near 0 and away
+// from it share the middle of their series (the terms from y^2/2 down to
+// y^8/8!), so lanes of both kinds run it once.
+STORM_HD float expm1_neg(float y) {
+  const bool near = y > -0.34657359f;
+  const float yc = y < -87.0f ? -87.0f : y;  // e^-87 - 1 rounds to -1
+  const float kf = yc * kLog2e;
+  const int k = near ? 0 : static_cast<int>(kf - 0.5f);
+  const float fk = static_cast<float>(k);
+  const float r = fma_f(-fk, kLn2Lo, fma_f(-fk, kLn2Hi, yc));  // y itself for k = 0
+  const float p9 = fma_f(r, 1.0f / 362880.0f, 1.0f / 40320.0f);
+  float p = near ? p9 : 1.0f / 40320.0f;
+  p = fma_f(r, p, 1.0f / 5040.0f);
+  p = fma_f(r, p, 1.0f / 720.0f);
+  p = fma_f(r, p, 1.0f / 120.0f);
+  p = fma_f(r, p, 1.0f / 24.0f);
+  p = fma_f(r, p, 1.0f / 6.0f);
+  p = fma_f(r, p, 0.5f);
+  const float small = fma_f(r * r, p, r);
+  const float q = fma_f(r, fma_f(r, p, 1.0f), 1.0f);
+  // 2^k is normal for k >= -126, and what is lost below 1 does not matter
+  const float big = q * u2f(static_cast<uint32_t>(k + 127) << 23) - 1.0f;
+  return near ? small : big;
 }
 
 // sin and cos of 2*pi*u for u in [0, 1].

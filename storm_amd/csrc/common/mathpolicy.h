@@ -19,7 +19,25 @@ template <>
 struct MathPolicy<float> {
   STORM_HD static float log(float x) { return fpm::logf_d(x); }
   STORM_HD static float exp(float x) { return fpm::expf_d(x); }
-  STORM_HD static float expm1(float x) { return fpm::expm1f_d(x); }
+  STORM_HD static float expm1_neg(float x) { return fpm::expm1_neg(x); }  // x <= 0
+  STORM_HD static float log_unit(float x) { return fpm::log_unit(x); }    // x a uniform or 1 minus one
+  STORM_HD static float recip(float x) { return fpm::recip_f(x); }        // |x| in [2^-126, 2^126]
+  STORM_HD static float recip_any(float x) {
+    return (x >= 0x1p-126f && x <= 0x1p126f) ? fpm::recip_f(x) : 1.0f / x;
+  }
+  // a / b, rounded as IEEE does for b within [2^-60, 2^60] and a 0 or within
+  // [2^-60, 2^60]; elsewhere about it, or no number
+  STORM_HD static float div_tame(float a, float b) { return fpm::div_f(a, b); }
+  // the middle one of three, the smaller of the others if one is no number
+  STORM_HD static float median(float a, float b, float c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_fmed3f(a, b, c);
+#else
+    const float lo = a < b ? a : b, hi = a < b ? b : a;
+    return c < lo ? lo : (c > hi ? hi : c);
+#endif
+  }
+  STORM_HD static float sqrt_unit(float x) { return fpm::sqrt_f(x); }     // x 0 or in [2^-100, 2^100]
   STORM_HD static void sincos2pi(float u, float &s, float &c) { fpm::sincos2pi(u, s, c); }
   STORM_HD static float sqrt(float x) { return ::sqrtf(x); }
   STORM_HD static float uniform(uint32_t x) { return u01_f32(x); }
@@ -30,7 +48,16 @@ template <>
 struct MathPolicy<double> {
   STORM_HD static double log(double x) { return ::log(x); }
   STORM_HD static double exp(double x) { return ::exp(x); }
-  STORM_HD static double expm1(double x) { return ::expm1(x); }
+  STORM_HD static double expm1_neg(double x) { return ::expm1(x); }
+  STORM_HD static double log_unit(double x) { return ::log(x); }
+  STORM_HD static double recip(double x) { return 1.0 / x; }
+  STORM_HD static double recip_any(double x) { return 1.0 / x; }
+  STORM_HD static double div_tame(double a, double b) { return a / b; }
+  STORM_HD static double median(double a, double b, double c) {
+    const double lo = a < b ? a : b, hi = a < b ? b : a;
+    return c < lo ? lo : (c > hi ? hi : c);
+  }
+  STORM_HD static double sqrt_unit(double x) { return ::sqrt(x); }
   STORM_HD static void sincos2pi(double u, double &s, double &c) {
     double a = 6.283185307179586476925286766559 * u;
     s = ::sin(a);

@@ -30,6 +30,15 @@ STORM_HD void mulhilo(uint32_t a, uint32_t b, uint32_t &hi, uint32_t &lo) {
   hi = static_cast<uint32_t>(p >> 32);
   lo = static_cast<uint32_t>(p);
 }
+
+// a ^ b ^ c (one instruction on gfx950)
+STORM_HD uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96);
+#else
+  return a ^ b ^ c;
+#endif
+}
 }  // namespace philox_detail
 
 // One Philox4x32 block with 10 rounds.
@@ -43,8 +52,8 @@ STORM_HD Philox4 philox4x32_10(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c
     uint32_t hi0, lo0, hi1, lo1;
     mulhilo(kM0, c0, hi0, lo0);
     mulhilo(kM1, c2, hi1, lo1);
-    uint32_t n0 = hi1 ^ c1 ^ k0;
-    uint32_t n2 = hi0 ^ c3 ^ k1;
+    uint32_t n0 = xor3(hi1, c1, k0);
+    uint32_t n2 = xor3(hi0, c3, k1);
     c0 = n0;
     c1 = lo1;
     c2 = n2;
@@ -60,9 +69,15 @@ STORM_HD Philox4 philox4x32_10(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c
   return out;
 }
 
-// (0,1) float from the top 24 bits of a word: (k + 0.5) * 2^-24.
+// (0,1) float from the top 24 bits of a word: (k + 0.5) * 2^-24, rounded once
+// (by the fused multiply-add; scaling by a power of two rounds nothing).
 STORM_HD float u01_f32(uint32_t x) {
-  return (static_cast<float>(x >> 8) + 0.5f) * 5.9604644775390625e-08f;
+  const float k = static_cast<float>(x >> 8);
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_fmaf(k, 5.9604644775390625e-08f, 2.98023223876953125e-08f);
+#else
+  return (k + 0.5f) * 5.9604644775390625e-08f;
+#endif
 }
 
 // (0,1) double from 53 bits of two words: (k + 0.5) * 2^-53.

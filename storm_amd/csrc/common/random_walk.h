@@ -66,8 +66,10 @@ STORM_HD Tables<Real> tables_at(const Real *all) {
 // S = 2 exp(-pi^2 T), gives T = (y + ln 2) / pi^2; the next mode is below
 // exp(-3 pi^2 T) < 2e-7 of it there.  Below the table (xi < 1.4e-11) T is
 // the first entry; xi = 1 gives kTauMax, as the reference's table end does.
+// `nlog` is -ln(1 - xi), which the trackers share with the other kinds of
+// step (any value where xi is below 1/64 or 1).
 template <typename Real>
-STORM_HD Real sample_leak_time(const Tables<Real> &t, Real xi) {
+STORM_HD Real sample_leak_time(const Tables<Real> &t, Real xi, Real nlog) {
   using M = MathPolicy<Real>;
   const Real s = Real(1) - xi;
   if (!(s > Real(0))) return Real(kTauMax);
@@ -75,7 +77,7 @@ STORM_HD Real sample_leak_time(const Tables<Real> &t, Real xi) {
   // since 1 - xi keeps too few of xi's bits in float
   const Real y = xi < Real(0.015625)
                      ? xi * (Real(1) + xi * (Real(0.5) + xi * (Real(1) / Real(3) + xi * (Real(0.25) + xi * Real(0.2)))))
-                     : -M::log(s);
+                     : nlog;
   const Real ly = y > Real(0) ? M::log(y) : Real(kLeakLogYMin);
   if (ly >= Real(kLeakLogYMax)) {
     const Real T = (y + Real(0.69314718055994530942)) * Real(0.10132118364233777144);  // 1 / pi^2
@@ -88,6 +90,12 @@ STORM_HD Real sample_leak_time(const Tables<Real> &t, Real xi) {
   const Real f = pos - static_cast<Real>(i);
   const Real t0 = t.leak[i], t1 = t.leak[i + 1];
   return t0 + f * (t1 - t0);
+}
+
+template <typename Real>
+STORM_HD Real sample_leak_time(const Tables<Real> &t, Real xi) {
+  const Real s = Real(1) - xi;
+  return sample_leak_time<Real>(t, xi, s > Real(0) ? -MathPolicy<Real>::log(s) : Real(0));
 }
 
 template <typename Real>

@@ -20,8 +20,9 @@
 // Layout (MI355X): a packet's position is kept relative to its cell's mesh
 // point (the Voronoi generator), so FP32 carries it to ~1e-7 of the cell
 // size; crossing a face adds the face's frame shift (mesh point of the cell
-// minus that of the neighbour).  Each face record is 32 bytes in FP32
-// (normal, plane offset in the cell's frame, neighbour, frame shift).
+// minus that of the neighbour).  Each face is 16 bytes of plane in FP32
+// (normal, offset in the cell's frame) and 32 of link (neighbour and its
+// faces, frame shift).
 #pragma once
 
 #include <stdint.h>
@@ -39,12 +40,34 @@ struct UFace {
   Real sh[3];    // mesh point of this cell minus that of the neighbour (0 on the box)
 };
 
+// The transport's two halves of a face: the plane, which every segment reads
+// for every face of its cell, and what only the face it leaves through needs,
+// with the neighbour's own planes [pbeg, pend) so that they are read without
+// looking them up in between.  A cell's planes are filled up to a multiple of
+// kFaceBatch with planes that nothing ever reaches (n = 0, d = +inf), so that
+// they are read and tried kFaceBatch at a time with no test for the last one;
+// links stand in the same places.
+constexpr uint32_t kFaceBatch = 3;
+template <typename Real>
+struct alignas(4 * sizeof(Real)) UPlane {
+  Real n[3], d;
+};
+template <typename Real>
+struct alignas(16) ULink {
+  int32_t nbr;
+  uint32_t pbeg, pend;
+  Real sh[3];
+};
+
 template <typename Real>
 struct UMeshView {
   uint32_t ncells;
   uint32_t escape_mask;            // bit s: box side s removes the packet (else it reflects)
   const uint32_t *face_start;      // ncells + 1
-  const UFace<Real> *face;         // per face
+  const uint32_t *plane_start;     // ncells + 1
+  const UPlane<Real> *plane;       // per face, filled up (kFaceBatch)
+  const ULink<Real> *link;         // per plane
+  uint32_t tame;                   // 1: every |d| lies in [2^-30, 2^50] (nearest_face)
   const Real *face_centroid;       // 3 per face, in the cell's frame (DDMC leaks)
   const Real *ddmc_rate;           // per face, leak rate / c (cm^-1); null without DDMC
   SpectrumView<Real> spec;
@@ -98,469 +121,389 @@ STORM_HD float umove_coord(float x, float nx, float delta, uint32_t r8) {
   return (static_cast<float>(r8) + 0.5f) * 0.00390625f < p ? up : x;
 }
 
-template <typename Real, uint32_t F = kFeatAll>
-struct UTracker {
-  using M = MathPolicy<Real>;
-  static constexpr bool fixed_point = sizeof(Real) == 4;
+// The faces of a cell are read kFaceBatch at a time (the loads of a batch
+// overlap; one face per turn waits for its load every time), in one pass that
+// gives the random walk's radius and the analytic step's nearest face alike.
+// The pass keeps the smallest distance and the second smallest; which face
+// the second belongs to matters only when the two nearly tie, and then the
+// faces are gone through again (resolve_tie).
 
-  PacketStream rs;
-  Real x0, x1, x2, o0, o1, o2, s, wmin, nu;
-  Real cell_sig_abs, cell_sig_ev, cell_sig_s, inv_sig_ev;
-  double w, w_enter, path_int;
-  uint32_t cell, ctr, visit_segs, id, fbeg, fend;
-  int outcome;
-  bool derive_pint;
-  // per-group tally (multigroup with withEgTimeAvg), as in Tracker
-  bool eg_track;
-  int32_t grp;
-  double eg_mark;
+template <typename Real, uint32_t F = kFeatAll>
+struct UTracker : PacketState<Real, F> {
+  using Base = PacketState<Real, F>;
+  using M = MathPolicy<Real>;
+  using Base::fixed_point;
+  using Base::multigroup;
+  using Base::o0;
+  using Base::o1;
+  using Base::o2;
+  using Base::s;
+  using Base::w;
+  using Base::wmin;
+  using Base::nu;
+  using Base::ctr;
+  using Base::id;
+  using Base::cell;
+  using Base::outcome;
+  using Base::cell_sig_abs;
+  using Base::cell_sig_ev;
+  using Base::cell_sig_s;
+  using Base::inv_sig_ev;
+
+  Real x0, x1, x2;
+  uint32_t pbeg, pend;  // the current cell's planes
 
   STORM_HD void begin(const Packet<Real> &p, const UMeshView<Real> &m, const CellXS<Real> *xs, const StepConsts &k) {
-    rs = PacketStream::make(k.seed, p.id, k.step, kTagTransport);
     x0 = p.u[0];
     x1 = p.u[1];
     x2 = p.u[2];
     o0 = p.o[0];
     o1 = p.o[1];
     o2 = p.o[2];
-    s = p.s;
-    w = p.w;
     cell = p.ijk;
-    ctr = p.ctr;
-    wmin = p.wmin;
-    id = p.id;
-    nu = p.nu;
-    eg_track = (F & kFeatMultigroup) != 0u && m.spec.groups >= 2 && m.spec.eg != 0;
-    grp = 0;
-    eg_mark = 0.0;
-    load_cell(m, xs);
-    w_enter = w;
-    path_int = 0.0;
-    visit_segs = 0;
-    outcome = kAlive;
+    pbeg = m.plane_start[cell];
+    pend = m.plane_start[cell + 1u];
+    this->begin_packet(p, m.spec, k);
+    this->set_opacity(m.spec, xs[cell], Base::is_mg(m.spec) ? m.spec.sig_s[cell] : Real(0));
   }
 
   template <typename Sink>
-  STORM_HD void end(Packet<Real> &p, const StepConsts &k, Sink &sink) {
-    if (outcome == kAlive) {
-      double wq = fixed_point ? fx::carry_round(w, w_enter, k.eq, id, ctr, cell) : w;
-      flush(wq, k, sink);
-      w = wq;
-    }
+  STORM_HD void end(Packet<Real> &p, const UMeshView<Real> &m, const StepConsts &k, Sink &sink) {
+    this->end_packet(p, m.spec, k, sink);
     p.u[0] = x0;
     p.u[1] = x1;
     p.u[2] = x2;
-    p.o[0] = o0;
-    p.o[1] = o1;
-    p.o[2] = o2;
-    p.s = s;
-    p.w = w;
-    p.wmin = wmin;
     p.ijk = cell;
-    p.ctr = ctr;
-    p.id = id;
-    p.nu = nu;
   }
 
-  STORM_HD bool derives_path_integral(const UMeshView<Real> &m) const {
-    if constexpr ((F & kFeatMultigroup) != 0u) {
-      if (m.spec.groups >= 2) return false;
+  // Whether (a0, a1, a2) lies within every face plane of the cell.
+  STORM_HD bool inside(const UMeshView<Real> &m, Real a0, Real a1, Real a2) const {
+    bool in = true;
+    for (uint32_t f = pbeg; f < pend && in; f += kFaceBatch) {
+      UPlane<Real> pl[kFaceBatch];
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma unroll
+#endif
+      for (uint32_t j = 0; j < kFaceBatch; ++j) pl[j] = m.plane[f + j];
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma unroll
+#endif
+      for (uint32_t j = 0; j < kFaceBatch; ++j)
+        in = in && pl[j].n[0] * a0 + pl[j].n[1] * a1 + pl[j].n[2] * a2 <= pl[j].d;
     }
-    return fixed_point && cell_sig_abs > Real(0);
+    return in;
   }
 
-  // Hands the path integral since the last call to the packet's group: at
-  // the end of each visit and before the photon energy changes.
-  template <typename Sink>
-  STORM_HD void group_split(const StepConsts &k, Sink &sink) {
-    if constexpr ((F & kFeatMultigroup) != 0u) {
-      if (eg_track) {
-        const double v = path_int - eg_mark;
-        if (v > 0.0) sink.group_path(cell, grp, v, k, group_tally_draw(id, ctr, cell, grp));
-        eg_mark = path_int;
-      }
-    }
-  }
-
-  template <typename Sink>
-  STORM_HD void flush(double w_exit, const StepConsts &k, Sink &sink) {
-    group_split(k, sink);
-    eg_mark = 0.0;
-    if constexpr (fixed_point) {
-      fx::Limbs d = fx::sub(fx::limbs_of(w_enter, k.eq), fx::limbs_of(w_exit, k.eq));
-      fx::Limbs e{0u, 0u};
-      if (!derive_pint) {
-        uint32_t h = id * 0x9E3779B1u ^ (ctr + 0x7F4A7C15u) * 0x85EBCA77u ^ cell * 0xC2B2AE3Du;
-        h ^= h >> 15;
-        h *= 0x2C1B3C6Du;
-        h ^= h >> 12;
-        e = fx::limbs_of(fx::quantize_unbiased(path_int, k.et, h >> 8), k.et);
-      }
-      sink.visit(cell, d, e, visit_segs);
-    } else {
-      sink.visit_fp(cell, w_enter - w_exit, path_int, visit_segs);
-    }
-    visit_segs = 0;
-    path_int = 0.0;
-  }
-
-  STORM_HD void load_cell(const UMeshView<Real> &m, const CellXS<Real> *xs) {
-    fbeg = m.face_start[cell];
-    fend = m.face_start[cell + 1u];
-    load_opacity(m, xs);
-  }
-  STORM_HD void load_opacity(const UMeshView<Real> &m, const CellXS<Real> *xs) {
-    const bool mg = (F & kFeatMultigroup) != 0u && m.spec.groups >= 2;
-    set_opacity(m, xs[cell], mg ? m.spec.sig_s[cell] : Real(0));
-  }
-  STORM_HD void set_opacity(const UMeshView<Real> &m, const CellXS<Real> &xc, Real sig_s) {
-    cell_sig_abs = xc.sig_abs;
-    cell_sig_ev = xc.sig_ev;
-    cell_sig_s = Real(0);
-    inv_sig_ev = xc.inv_ev;
-    if ((F & kFeatMultigroup) != 0u && m.spec.groups >= 2) {
-      Real e = nu < m.spec.e_lo ? m.spec.e_lo : (nu > m.spec.e_hi ? m.spec.e_hi : nu);
-      const Real fac = M::exp(-m.spec.nu_pow * M::log(e));
-      cell_sig_s = sig_s;
-      cell_sig_abs = xc.sig_abs * fac;
-      cell_sig_ev = cell_sig_s + xc.sig_ev * fac;
-      if (eg_track) grp = group_of<Real>(e, m.spec.bounds, m.spec.groups);
-      inv_sig_ev = cell_sig_ev > Real(0) ? Real(1) / cell_sig_ev : Real(0);
-    } else if constexpr ((F & kFeatAccel) != 0u) {
-      // the same value, divided here: loading it made the register
-      // allocation of the gray random-walk/DDMC kernel spill more (18%
-      // slower on the batch of slabs, measured)
-      inv_sig_ev = cell_sig_ev > Real(0) ? Real(1) / cell_sig_ev : Real(0);
-    }
-    derive_pint = derives_path_integral(m);
-  }
-
-  STORM_HD void absorb(Real sig_abs, Real d, bool tally_free) {
-    Real xabs = sig_abs * d;
-    Real frac = -M::expm1(-xabs);
-    double w0 = w;
-    w = w0 - w0 * static_cast<double>(frac);
-    if (derive_pint) return;
-    if (xabs >= Real(1e-12)) {
-      path_int += w0 * static_cast<double>(frac / sig_abs);
-    } else if (tally_free) {
-      path_int += w0 * static_cast<double>(d);
-    } else if (sig_abs > Real(0)) {
-      path_int += w0 * static_cast<double>(frac / sig_abs);
-    }
-  }
-
-  template <typename Sink>
-  STORM_HD void roulette(const StepConsts &k, Sink &sink) {
-    double wq = fixed_point ? fx::quantize_down(w, k.eq) : w;
-    flush(fixed_point ? wq : 0.0, k, sink);
-    if constexpr (fixed_point) sink.roulette(cell, wq);
-    w = 0.0;
-    outcome = kGone;
-  }
-
-  template <typename Sink>
-  STORM_HD void census(const StepConsts &k, Sink &sink) {
-    double wq = fx::carry_round(w, w_enter, k.eq, id, ctr, cell);
-    flush(wq, k, sink);
-    w = wq;
-    outcome = kCensus;
-  }
-
-  // Close the visit and continue in the cell across face `f`.
-  template <typename Sink>
-  STORM_HD void cross(const UFace<Real> &fc, const UMeshView<Real> &m, const CellXS<Real> *xs, const StepConsts &k,
-                      Sink &sink) {
-    double wq = fixed_point ? fx::carry_round(w, w_enter, k.eq, id, ctr, cell) : w;
-    flush(wq, k, sink);
-    w = wq;
-    w_enter = wq;
-    x0 += fc.sh[0];
-    x1 += fc.sh[1];
-    x2 += fc.sh[2];
-    cell = static_cast<uint32_t>(fc.nbr);
-    load_cell(m, xs);
-  }
-
-  template <typename Sink>
-  STORM_HD int segment(const UMeshView<Real> &m, const CellXS<Real> *xs, const AccelView<Real> &acc,
-                       const StepConsts &k, Sink &sink) {
-    const Real sig_abs = cell_sig_abs;
-    ++visit_segs;
-    if ((F & kFeatAccel) != 0u && acc.cell) {
-      const CellAccel<Real> ca = acc.cell[cell];
-      if (ca.flags) {
-        // distance to the nearest face plane (computeMinDistanceToFaces)
-        Real Ro = M::inf();
-        for (uint32_t f = fbeg; f < fend; ++f) {
-          const UFace<Real> fc = m.face[f];
-          const Real dist = fc.d - (fc.n[0] * x0 + fc.n[1] * x1 + fc.n[2] * x2);
-          Ro = dist < Ro ? dist : Ro;
-        }
-        if (!(Ro > Real(0))) Ro = Real(0);
-        const Real tauR = Ro * ca.sig_t;
-        const bool pgrw = (F & kFeatMultigroup) != 0u && m.spec.groups >= 2;
-        const bool walks = !pgrw || nu < ca.e_cut;
-        if ((ca.flags & 1u) && walks && Ro > Real(0) && ca.sig_t > Real(0) && tauR >= acc.rw_particle_tau) {
-          // ---------------- random-walk step (tryRandomWalkStep)
-          const Philox4 r = rs.block(ctr++);
-          const Philox4 r2 = rs.block(ctr++);
-          const rw::Tables<Real> tb = rw::tables_at(acc.rw);
-          const Real tauLeak = rw::sample_leak_time<Real>(tb, M::uniform(r.v[0]));
-          const Real sig_d = pgrw ? ca.sig_d : ca.sig_t;
-          const Real sLeak = tauLeak * Ro * Ro * (Real(3) * sig_d);
-          Real sUp = M::inf();
-          if (pgrw && ca.up_rate > Real(0)) sUp = (-M::log(M::uniform(r2.v[2]))) / ca.up_rate;
-          int rev = 0;
-          Real d = sLeak;
-          if (!(sLeak <= s && sLeak <= sUp)) {
-            rev = s <= sUp ? 1 : 2;
-            d = rev == 1 ? s : sUp;
-          }
-          const bool leak = rev == 0;
-          absorb(pgrw ? ca.sig_abs : sig_abs, d, false);
-          s = rev == 1 ? Real(0) : s - d;
-          if (s < Real(0)) s = Real(0);
-          sink.rw_step();
-          if (w < static_cast<double>(wmin * Real(0.1))) {
-            roulette(k, sink);
-            return outcome;
-          }
-          Real dir[3];
-          isotropic_dir<Real>(M::uniform(r.v[1]), M::uniform(r.v[2]), dir);
-          Real disp = Ro;
-          if (!leak) {
-            const Real tauPos = d / (Real(3) * sig_d * Ro * Ro);
-            disp = Ro * rw::sample_radius<Real>(tb, tauPos, M::uniform(r.v[3]));
-          }
-          if (disp > Ro) disp = Ro;
-          const Real c0 = x0, c1 = x1, c2 = x2;
-          // nudge towards the mesh point, the frame's origin (:1214-1215)
-          Real n0 = (c0 + disp * dir[0]) * Real(1 - 1e-6);
-          Real n1 = (c1 + disp * dir[1]) * Real(1 - 1e-6);
-          Real n2 = (c2 + disp * dir[2]) * Real(1 - 1e-6);
-          for (int guard = 0; guard < 2000; ++guard) {
-            bool inside = true;
-            for (uint32_t f = fbeg; f < fend && inside; ++f) {
-              const UFace<Real> fc = m.face[f];
-              inside = fc.n[0] * n0 + fc.n[1] * n1 + fc.n[2] * n2 <= fc.d;
-            }
-            if (inside) break;
-            disp = disp * Real(0.99);
-            n0 = c0 + disp * dir[0];
-            n1 = c1 + disp * dir[1];
-            n2 = c2 + disp * dir[2];
-          }
-          x0 = n0;
-          x1 = n1;
-          x2 = n2;
-          Real nd[3];
-          isotropic_dir<Real>(M::uniform(r2.v[0]), M::uniform(r2.v[1]), nd);
-          o0 = nd[0];
-          o1 = nd[1];
-          o2 = nd[2];
-          if ((F & kFeatMultigroup) != 0u && rev == 2) {
-            const int32_t G = m.spec.groups;
-            const Real *cdfc = m.spec.cdf + static_cast<size_t>(cell) * static_cast<size_t>(G + 1);
-            const Real lo = cdfc[ca.gcut];
-            group_split(k, sink);
-            if (lo < Real(1)) {
-              nu = spectrum_quantile<Real>(cdfc, m.spec.bounds, G, lo + M::uniform(r2.v[3]) * (Real(1) - lo));
-            } else {
-              nu = next_above(m.spec.bounds[ca.gcut]);
-            }
-            nu = nu < m.spec.e_lo ? m.spec.e_lo : (nu > m.spec.e_hi ? m.spec.e_hi : nu);
-            load_opacity(m, xs);
-          }
-          if (rev == 1) census(k, sink);
-          return outcome;
-        }
-        if ((ca.flags & 2u) && ca.total > Real(0) && Ro * ca.ddmc_sig_t >= acc.ddmc_particle_tau &&
-            ((F & kFeatMultigroup) == 0u || nu < ca.ddmc_e_cut) && m.ddmc_rate) {
-          // ---------------- DDMC step (tryDDMCStep)
-          const Philox4 r = rs.block(ctr++);
-          const Real sEvent = (-M::log(M::uniform(r.v[0]))) / ca.total;
-          const bool cen = s <= sEvent;
-          const Real d = cen ? s : sEvent;
-          absorb((F & kFeatMultigroup) != 0u ? ca.ddmc_abs : sig_abs, d, true);
-          s = cen ? Real(0) : s - d;
-          if (s < Real(0)) s = Real(0);
-          sink.ddmc_step();
-          if (w < static_cast<double>(wmin)) {
-            roulette(k, sink);
-            return outcome;
-          }
-          if (cen) {
-            census(k, sink);
-            return outcome;
-          }
-          // leak through a face chosen in proportion to its rate
-          Real pick = M::uniform(r.v[1]) * ca.total;
-          uint32_t face = 0xFFFFFFFFu, lastf = 0xFFFFFFFFu;
-          for (uint32_t f = fbeg; f < fend; ++f) {
-            const Real rt = m.ddmc_rate[f];
-            if (rt > Real(0)) {
-              lastf = f;
-              pick -= rt;
-              if (face == 0xFFFFFFFFu && pick <= Real(0)) face = f;
-            }
-          }
-          if (face == 0xFFFFFFFFu) face = lastf;
-          const UFace<Real> fc = m.face[face];
-          // mu = sqrt(U) about the outward normal, basis as in :1565-1586
-          const Real mu = M::sqrt(M::uniform(r.v[2]));
-          const Real st2 = Real(1) - mu * mu;
-          const Real st = M::sqrt(st2 > Real(0) ? st2 : Real(0));
-          Real sp, cp;
-          M::sincos2pi(M::uniform(r.v[3]), sp, cp);
-          const Real nx = fc.n[0], ny = fc.n[1], nz = fc.n[2];
-          const bool hx = (nx < Real(0) ? -nx : nx) < Real(0.9);
-          // helper (1,0,0) or (0,1,0), e1 = helper - (helper . n) n, e2 = n x e1
-          Real e10 = (hx ? Real(1) : Real(0)) - (hx ? nx : ny) * nx;
-          Real e11 = (hx ? Real(0) : Real(1)) - (hx ? nx : ny) * ny;
-          Real e12 = -(hx ? nx : ny) * nz;
-          const Real e1n = M::sqrt(e10 * e10 + e11 * e11 + e12 * e12);
-          if (e1n > Real(0)) {
-            e10 /= e1n;
-            e11 /= e1n;
-            e12 /= e1n;
-          }
-          const Real e20 = ny * e12 - nz * e11, e21 = nz * e10 - nx * e12, e22 = nx * e11 - ny * e10;
-          Real d0 = mu * nx + st * cp * e10 + st * sp * e20;
-          Real d1 = mu * ny + st * cp * e11 + st * sp * e21;
-          Real d2 = mu * nz + st * cp * e12 + st * sp * e22;
-          const Real dn = M::sqrt(d0 * d0 + d1 * d1 + d2 * d2);
-          if (dn > Real(0)) {
-            d0 /= dn;
-            d1 /= dn;
-            d2 /= dn;
-          }
-          o0 = d0;
-          o1 = d1;
-          o2 = d2;
-          // on the face centroid (:1588), then into the neighbour
-          x0 = m.face_centroid[3 * face];
-          x1 = m.face_centroid[3 * face + 1];
-          x2 = m.face_centroid[3 * face + 2];
-          cross(fc, m, xs, k, sink);
-          return outcome;
-        }
-      }
-    }
-
-    // ---------------- analytic step
-    // nearest face along the direction, and the next one for ties
-    Real dface = M::inf(), dsecond = M::inf();
-    uint32_t fa = fbeg, fb = fbeg;
-    for (uint32_t f = fbeg; f < fend; ++f) {
-      const UFace<Real> fc = m.face[f];
+  // Two faces at (nearly) the smallest distance: the nearest and the next one
+  // in the order of the faces, and, in the mixed engine, when they are within
+  // 1e-6 along the path (an edge or a vertex), the choice between them in FP64.
+  STORM_HD void resolve_tie(const UMeshView<Real> &m, Real &d, uint32_t &fa) const {
+    Real dsecond = M::inf();
+    uint32_t fb = pbeg;
+    d = M::inf();
+    fa = pbeg;
+    for (uint32_t f = pbeg; f < pend; ++f) {
+      const UPlane<Real> fc = m.plane[f];
       const Real den = fc.n[0] * o0 + fc.n[1] * o1 + fc.n[2] * o2;
       if (!(den > Real(0))) continue;
       Real t = (fc.d - (fc.n[0] * x0 + fc.n[1] * x1 + fc.n[2] * x2)) / den;
       t = t > Real(0) ? t : Real(0);
-      if (t < dface) {
-        dsecond = dface;
+      if (t < d) {
+        dsecond = d;
         fb = fa;
-        dface = t;
+        d = t;
         fa = f;
       } else if (t < dsecond) {
         dsecond = t;
         fb = f;
       }
     }
-    if constexpr (fixed_point) {
-      // two faces within 1e-6 along the path (an edge or a vertex): decide in FP64
-      if (dsecond < M::inf() && dsecond - dface <= Real(1e-6) * dsecond) {
-        auto dist64 = [&](uint32_t f) {
-          const UFace<Real> fc = m.face[f];
-          const double den = static_cast<double>(fc.n[0]) * o0 + static_cast<double>(fc.n[1]) * o1 +
-                             static_cast<double>(fc.n[2]) * o2;
-          const double num = static_cast<double>(fc.d) - (static_cast<double>(fc.n[0]) * x0 +
-                                                          static_cast<double>(fc.n[1]) * x1 +
-                                                          static_cast<double>(fc.n[2]) * x2);
-          const double t = num / den;
-          return t > 0.0 ? t : 0.0;
-        };
-        const double dA = dist64(fa), dB = dist64(fb);
-        if (dB < dA) {
-          fa = fb;
-          dface = static_cast<Real>(dB);
-        }
+    if (fixed_point && dsecond < M::inf() && dsecond - d <= Real(1e-6) * dsecond) {
+      auto dist64 = [&](uint32_t f) {
+        const UPlane<Real> fc = m.plane[f];
+        const double den = static_cast<double>(fc.n[0]) * o0 + static_cast<double>(fc.n[1]) * o1 +
+                           static_cast<double>(fc.n[2]) * o2;
+        const double num = static_cast<double>(fc.d) - (static_cast<double>(fc.n[0]) * x0 +
+                                                        static_cast<double>(fc.n[1]) * x1 +
+                                                        static_cast<double>(fc.n[2]) * x2);
+        const double t = num / den;
+        return t > 0.0 ? t : 0.0;
+      };
+      const double dA = dist64(fa), dB = dist64(fb);
+      if (dB < dA) {
+        fa = fb;
+        d = static_cast<Real>(dB);
       }
     }
-    const UFace<Real> fcx = m.face[fa];
-    const Philox4 r = rs.block(ctr++);
-    Real xi = M::uniform(r.v[0]);
-    Real dcol = cell_sig_ev > Real(0) ? (-M::log(xi)) * inv_sig_ev : M::inf();
-    int ev = 0;
-    Real d = dface;
-    if (dcol < d) {
-      ev = 1;
-      d = dcol;
+  }
+
+  template <typename Sink>
+  STORM_HD int segment(const UMeshView<Real> &m, const CellXS<Real> *xs, const AccelView<Real> &acc,
+                       const StepConsts &k, Sink &sink) {
+    const PacketStream rs = PacketStream::make(k.seed, id, k.step, kTagTransport);
+    const bool mg = Base::is_mg(m.spec);
+    ++this->visit_segs;
+
+    // ---------------- the distance to the nearest face plane
+    // (computeMinDistanceToFaces), and along the direction to the nearest
+    // face and the next one for ties
+    Real Ro = M::inf();
+    Real d = M::inf(), dsecond = M::inf();
+    uint32_t fa = 0u;
+    for (uint32_t f = pbeg; f < pend; f += kFaceBatch) {
+      UPlane<Real> pl[kFaceBatch];
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma unroll
+#endif
+      for (uint32_t j = 0; j < kFaceBatch; ++j) pl[j] = m.plane[f + j];
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma unroll
+#endif
+      for (uint32_t j = 0; j < kFaceBatch; ++j) {
+        const UPlane<Real> &fc = pl[j];
+        const Real dist = fc.d - (fc.n[0] * x0 + fc.n[1] * x1 + fc.n[2] * x2);
+        if constexpr ((F & kFeatAccel) != 0u) Ro = dist < Ro ? dist : Ro;
+        const Real den = fc.n[0] * o0 + fc.n[1] * o1 + fc.n[2] * o2;
+        // 0 where the packet sits on or beyond the face.  On a tame mesh a
+        // positive distance is above 2^-56 (it is a multiple of a unit of d)
+        // and a denominator below 2^-60 only ever makes a face too far to
+        // matter, so the short division is exact where it counts.
+        const Real a = dist > Real(0) ? dist : Real(0);
+        Real t = m.tame ? M::div_tame(a, den) : a / den;
+        t = den > Real(0) ? t : M::inf();
+        fa = t < d ? f + j : fa;
+        dsecond = M::median(d, dsecond, t);
+        d = t < d ? t : d;
+      }
     }
-    if (s < d) {
-      ev = 2;
+
+    // ---------------- which kind of step (CellXS::r_acc as on the Cartesian mesh)
+    int step = kStepAnalytic;
+    if constexpr ((F & kFeatAccel) != 0u) {
+      if (!(Ro > Real(0))) Ro = Real(0);
+      if (acc.cell && Ro >= this->r_acc) {
+        const CellAccel<Real> &ca = acc.cell[cell];
+        if ((ca.flags & 1u) && (!mg || nu < ca.e_cut) && Ro > Real(0) && ca.sig_t > Real(0) &&
+            Ro * ca.sig_t >= acc.rw_particle_tau)
+          step = kStepWalk;
+        else if ((ca.flags & 2u) && ca.total > Real(0) && Ro * ca.ddmc_sig_t >= acc.ddmc_particle_tau &&
+                 (!multigroup || nu < ca.ddmc_e_cut) && m.ddmc_rate)
+          step = kStepDdmc;
+      }
+    }
+    ULink<Real> ln{};
+    if (step == kStepAnalytic) {
+      // (also when no face lies ahead, or a denominator was too small a number)
+      if (fixed_point && !(dsecond - d > Real(1e-6) * dsecond)) resolve_tie(m, d, fa);
+      ln = m.link[fa];
+    }
+
+    // ---------------- random numbers (as Tracker::segment)
+    Philox4 r = rs.block(ctr++);
+    const Real xi = M::uniform(r.v[0]);
+    const Real nlog = -M::log_unit(step == kStepWalk ? Real(1) - xi : xi);
+
+    // ---------------- the event (d: its distance)
+    int ev = kEvFace;
+    Real sig_abs = cell_sig_abs;
+    Philox4 r2{};
+    if (step == kStepAnalytic) {
+      const Real dcol = cell_sig_ev > Real(0) ? nlog * inv_sig_ev : M::inf();
+      if (dcol < d) {
+        ev = kEvCollide;
+        d = dcol;
+      }
+    } else if ((F & kFeatAccel) != 0u && step == kStepWalk) {
+      // random-walk step (tryRandomWalkStep)
+      const CellAccel<Real> &ca = acc.cell[cell];
+      r2 = rs.block(ctr++);
+      const Real tauLeak = rw::sample_leak_time<Real>(rw::tables_at(acc.rw), xi, nlog);
+      d = tauLeak * Ro * Ro * (Real(3) * (mg ? ca.sig_d : ca.sig_t));
+      ev = kEvLeak;
+      if (mg) {
+        sig_abs = ca.sig_abs;
+        if (ca.up_rate > Real(0)) {
+          const Real sUp = (-M::log(M::uniform(r2.v[2]))) / ca.up_rate;
+          if (sUp < d && sUp < s) {
+            ev = kEvReemit;
+            d = sUp;
+          }
+        }
+      }
+    } else if constexpr ((F & kFeatAccel) != 0u) {
+      // DDMC step (tryDDMCStep)
+      const CellAccel<Real> &ca = acc.cell[cell];
+      d = nlog / ca.total;
+      ev = kEvLeak;
+      if constexpr (multigroup) sig_abs = ca.ddmc_abs;
+    }
+    if (s < d || (step == kStepDdmc && s == d)) {
+      ev = kEvCensus;
       d = s;
     }
-    s -= d;
-    if (ev == 2 || s < Real(0)) s = Real(0);
 
-    absorb(sig_abs, d, true);
-    {
+    this->absorb(m.spec, sig_abs, d, step != kStepWalk);
+    s = ev == kEvCensus ? Real(0) : s - d;
+    if (s < Real(0)) s = Real(0);
+    if constexpr ((F & kFeatAccel) != 0u) {
+      if (step == kStepWalk) sink.rw_step();
+      if (step == kStepDdmc) sink.ddmc_step();
+    }
+
+    int end = ev == kEvCensus ? kEndCensus : kEndNone;
+    bool turn = false;
+    Real fn0 = Real(0), fn1 = Real(0), fn2 = Real(0);  // DDMC: the leak face's normal
+    if (w < static_cast<double>(step == kStepWalk ? wmin * Real(0.1) : wmin)) {
+      end = kEndRoulette;
+    } else if (step == kStepAnalytic) {
       const Real m0 = o0 * d, m1 = o1 * d, m2 = o2 * d;
       Real n0 = x0 + m0, n1 = x1 + m1, n2 = x2 + m2;
       if constexpr (fixed_point) {
-        n0 = umove_coord(x0, n0, m0, r.v[1] & 0xffu);
-        n1 = umove_coord(x1, n1, m1, r.v[2] & 0xffu);
-        n2 = umove_coord(x2, n2, m2, r.v[3] & 0xffu);
+        if (n0 == x0 || n1 == x1 || n2 == x2) {
+          n0 = umove_coord(x0, n0, m0, r.v[1] & 0xffu);
+          n1 = umove_coord(x1, n1, m1, r.v[2] & 0xffu);
+          n2 = umove_coord(x2, n2, m2, r.v[3] & 0xffu);
+        }
       }
       x0 = n0;
       x1 = n1;
       x2 = n2;
-    }
-    if (w < static_cast<double>(wmin)) {
-      roulette(k, sink);
-      return outcome;
-    }
-    if (ev == 0) {
-      if (fcx.nbr >= 0) {
-        cross(fcx, m, xs, k, sink);
+      if (ev == kEvCollide) {
+        turn = true;
+        if (mg && !(M::uniform(r.v[1]) * cell_sig_ev < cell_sig_s)) ev = kEvReemit;
+      } else if (ev == kEvCensus) {
+      } else if (ln.nbr >= 0) {
+        end = kEndCross;
+      } else if ((m.escape_mask >> static_cast<uint32_t>(-1 - ln.nbr)) & 1u) {
+        end = kEndEscape;
       } else {
-        const uint32_t side = static_cast<uint32_t>(-1 - fcx.nbr);
-        if ((m.escape_mask >> side) & 1u) {
-          double wq = fixed_point ? fx::carry_round(w, w_enter, k.eq, id, ctr, cell) : w;
-          flush(wq, k, sink);
-          if constexpr (fixed_point) sink.escape_fx(cell, wq);
-          else sink.escape_fp(cell, wq);
-          w = 0.0;
-          outcome = kEscaped;
-        } else {
-          // specular reflection on the box face (BoundaryCondition.hpp:87-108)
-          const Real on = o0 * fcx.n[0] + o1 * fcx.n[1] + o2 * fcx.n[2];
-          o0 -= Real(2) * on * fcx.n[0];
-          o1 -= Real(2) * on * fcx.n[1];
-          o2 -= Real(2) * on * fcx.n[2];
+        // specular reflection on the box face (BoundaryCondition.hpp:87-108)
+        const UPlane<Real> fc = m.plane[fa];
+        const Real on = o0 * fc.n[0] + o1 * fc.n[1] + o2 * fc.n[2];
+        o0 -= Real(2) * on * fc.n[0];
+        o1 -= Real(2) * on * fc.n[1];
+        o2 -= Real(2) * on * fc.n[2];
+      }
+    } else if ((F & kFeatAccel) != 0u && step == kStepWalk) {
+      Real dir[3];
+      isotropic_dir<Real>(M::uniform(r.v[1]), M::uniform(r.v[2]), dir);
+      Real disp = Ro;
+      if (ev != kEvLeak) {
+        const Real sig_d = mg ? acc.cell[cell].sig_d : acc.cell[cell].sig_t;
+        const Real tauPos = d / (Real(3) * sig_d * Ro * Ro);
+        disp = Ro * rw::sample_radius<Real>(rw::tables_at(acc.rw), tauPos, M::uniform(r.v[3]));
+      }
+      if (disp > Ro) disp = Ro;
+      const Real c0 = x0, c1 = x1, c2 = x2;
+      // nudge towards the mesh point, the frame's origin (:1214-1215)
+      Real n0 = (c0 + disp * dir[0]) * Real(1 - 1e-6);
+      Real n1 = (c1 + disp * dir[1]) * Real(1 - 1e-6);
+      Real n2 = (c2 + disp * dir[2]) * Real(1 - 1e-6);
+      for (int guard = 0; guard < 2000; ++guard) {
+        if (inside(m, n0, n1, n2)) break;
+        disp = disp * Real(0.99);
+        n0 = c0 + disp * dir[0];
+        n1 = c1 + disp * dir[1];
+        n2 = c2 + disp * dir[2];
+      }
+      x0 = n0;
+      x1 = n1;
+      x2 = n2;
+      turn = true;
+      r.v[2] = r2.v[0];
+      r.v[3] = r2.v[1];
+    } else if ((F & kFeatAccel) != 0u && ev == kEvLeak) {
+      // DDMC leak through a face chosen in proportion to its rate
+      Real pick = M::uniform(r.v[1]) * acc.cell[cell].total;
+      uint32_t face = 0xFFFFFFFFu, lastf = 0xFFFFFFFFu;
+      const uint32_t fbeg = m.face_start[cell], fend = m.face_start[cell + 1u];
+      for (uint32_t f = fbeg; f < fend; ++f) {
+        const Real rt = m.ddmc_rate[f];
+        if (rt > Real(0)) {
+          lastf = f;
+          pick -= rt;
+          if (face == 0xFFFFFFFFu && pick <= Real(0)) face = f;
         }
       }
-    } else if (ev == 1) {
-      Real nd[3];
-      isotropic_dir<Real>(M::uniform(r.v[2]), M::uniform(r.v[3]), nd);
-      o0 = nd[0];
-      o1 = nd[1];
-      o2 = nd[2];
-      if ((F & kFeatMultigroup) != 0u && m.spec.groups >= 2) {
-        const bool elastic = M::uniform(r.v[1]) * cell_sig_ev < cell_sig_s;
-        if (!elastic) {
-          group_split(k, sink);
-          const Philox4 r2 = rs.block(ctr++);
-          const int32_t G = m.spec.groups;
-          nu = spectrum_quantile<Real>(m.spec.cdf + static_cast<size_t>(cell) * static_cast<size_t>(G + 1),
-                                       m.spec.bounds, G, M::uniform(r2.v[0]));
-          load_opacity(m, xs);
+      if (face == 0xFFFFFFFFu) face = lastf;
+      const UPlane<Real> fc = m.plane[pbeg + (face - fbeg)];
+      fn0 = fc.n[0];
+      fn1 = fc.n[1];
+      fn2 = fc.n[2];
+      ln = m.link[pbeg + (face - fbeg)];
+      // on the face centroid (:1588), then into the neighbour
+      x0 = m.face_centroid[3 * face];
+      x1 = m.face_centroid[3 * face + 1];
+      x2 = m.face_centroid[3 * face + 2];
+      turn = true;
+      end = kEndCross;
+    }
+
+    // ---------------- new direction: isotropic, or (a DDMC leak) mu = sqrt(U)
+    // about the outward normal, basis as in :1565-1586
+    if (turn) {
+      const bool ddmc = (F & kFeatAccel) != 0u && step == kStepDdmc;
+      const Real ua = M::uniform(r.v[2]), ub = M::uniform(r.v[3]);
+      const Real mu = ddmc ? M::sqrt_unit(ua) : Real(2) * ua - Real(1);
+      const Real st2 = Real(1) - mu * mu;
+      const Real st = M::sqrt_unit(st2 > Real(0) ? st2 : Real(0));
+      Real sp, cp;
+      M::sincos2pi(ub, sp, cp);
+      const Real x = st * cp, y = st * sp;
+      o0 = x;
+      o1 = y;
+      o2 = mu;
+      if (ddmc) {
+        const Real nx = fn0, ny = fn1, nz = fn2;
+        const bool hx = (nx < Real(0) ? -nx : nx) < Real(0.9);
+        // helper (1,0,0) or (0,1,0), e1 = helper - (helper . n) n, e2 = n x e1
+        Real e10 = (hx ? Real(1) : Real(0)) - (hx ? nx : ny) * nx;
+        Real e11 = (hx ? Real(0) : Real(1)) - (hx ? nx : ny) * ny;
+        Real e12 = -(hx ? nx : ny) * nz;
+        const Real e1n = M::sqrt(e10 * e10 + e11 * e11 + e12 * e12);
+        if (e1n > Real(0)) {
+          e10 /= e1n;
+          e11 /= e1n;
+          e12 /= e1n;
         }
+        const Real e20 = ny * e12 - nz * e11, e21 = nz * e10 - nx * e12, e22 = nx * e11 - ny * e10;
+        Real d0 = mu * nx + x * e10 + y * e20;
+        Real d1 = mu * ny + x * e11 + y * e21;
+        Real d2 = mu * nz + x * e12 + y * e22;
+        const Real dn = M::sqrt(d0 * d0 + d1 * d1 + d2 * d2);
+        if (dn > Real(0)) {
+          d0 /= dn;
+          d1 /= dn;
+          d2 /= dn;
+        }
+        o0 = d0;
+        o1 = d1;
+        o2 = d2;
       }
-    } else {
-      census(k, sink);
+    }
+    if constexpr (multigroup) {
+      if (ev == kEvReemit && end == kEndNone) {
+        this->group_split(m.spec, k, sink);
+        const bool walk = (F & kFeatAccel) != 0u && step == kStepWalk;
+        const Philox4 re = rs.block(walk ? ctr - 1u : ctr);
+        if (!walk) ++ctr;
+        this->new_energy(m.spec, M::uniform(walk ? re.v[3] : re.v[0]), walk ? acc.cell[cell].gcut : 0u);
+        this->set_opacity(m.spec, xs[cell], m.spec.sig_s[cell]);
+      }
+    }
+
+    // ---------------- the visit's end
+    if (end != kEndNone) {
+      this->end_visit(end, m.spec, k, sink);
+      if (end == kEndCross) {
+        x0 += ln.sh[0];
+        x1 += ln.sh[1];
+        x2 += ln.sh[2];
+        cell = static_cast<uint32_t>(ln.nbr);
+        pbeg = ln.pbeg;
+        pend = ln.pend;
+        this->set_opacity(m.spec, xs[cell], mg ? m.spec.sig_s[cell] : Real(0));
+      }
     }
     return outcome;
   }
@@ -577,7 +520,7 @@ STORM_HD int transport_packet(Packet<Real> &p, const UMeshView<Real> &m, const C
   UTracker<Real, F> t;
   t.begin(p, m, xs, k);
   for (int seg = 0; seg < max_segments && t.outcome == kAlive; ++seg) t.segment(m, xs, acc, k, sink);
-  t.end(p, k, sink);
+  t.end(p, m, k, sink);
   return t.outcome;
 }
 

@@ -10,6 +10,7 @@
 #include <cstdio>
 #include <cstring>
 #include <initializer_list>
+#include <limits>
 #include <type_traits>
 #include <memory>
 #include <mutex>
@@ -272,10 +273,7 @@ struct Engine final : EngineBase {
   DevBuf<uint32_t> vals, vals_out;  // comb: census indices sorted with the keys
   DevBuf<unsigned long long> tally_u64, emit_limbs, requant, leaving;
   DevBuf<double> tally_f64;
-  // per-XCD replicas 1..kTallyReplicas-1 of the per-visit tallies
-  DevBuf<unsigned long long> rep_u64;
-  DevBuf<double> rep_f64;
-  DevBuf<uint32_t> rep_u32;
+  DevBuf<unsigned long long> rec;  // Tallies::rec
   DevBuf<uint64_t> limbs_sorted, cum;  // sorted census weights in quanta, their prefix sums
   DevBuf<double> wsorted;              // sorted census weights
   DevBuf<CombCell> comb_cells;
@@ -318,7 +316,11 @@ struct Engine final : EngineBase {
   std::vector<double> chord_h;  // mean chord 4 V / S per cell
   DevBuf<double> chord;
   DevBuf<uint32_t> u_face_start, u_tet_start;
-  DevBuf<UFace<Real>> u_face;
+  DevBuf<UPlane<Real>> u_plane;
+  DevBuf<ULink<Real>> u_link;
+  DevBuf<uint32_t> u_plane_start;
+  DevBuf<int32_t> u_face_nbr;
+  bool u_tame = true;
   DevBuf<Real> u_face_centroid, u_ddmc_rate;
   DevBuf<double2> u_face_geo;
   DevBuf<UTet<Real>> u_tets;
@@ -557,7 +559,32 @@ struct Engine final : EngineBase {
         if (!h.empty()) HIPCHECK(hipMemcpy(d.p, h.data(), h.size() * sizeof(h[0]), hipMemcpyHostToDevice));
       };
       upv(u_face_start, ut.face_start);
-      upv(u_face, ut.face);
+      // planes and links, each cell's filled up to a multiple of kFaceBatch
+      std::vector<uint32_t> pstart(static_cast<size_t>(N) + 1);
+      for (uint32_t c = 0; c < N; ++c) {
+        const uint64_t n = ut.face_start[c + 1] - ut.face_start[c];
+        const uint64_t end = pstart[c] + (n + kFaceBatch - 1) / kFaceBatch * kFaceBatch;
+        if (end > 0xFFFFFFFFull) throw EngineError(1, "unstructured mesh: too many faces");
+        pstart[c + 1] = static_cast<uint32_t>(end);
+      }
+      const Real far = std::numeric_limits<Real>::infinity();
+      std::vector<UPlane<Real>> plane(pstart[N], UPlane<Real>{{Real(0), Real(0), Real(0)}, far});
+      std::vector<ULink<Real>> link(pstart[N], ULink<Real>{});
+      std::vector<int32_t> nbr(ut.face.size());
+      for (uint32_t c = 0; c < N; ++c)
+        for (uint32_t f = ut.face_start[c], q = pstart[c]; f < ut.face_start[c + 1]; ++f, ++q) {
+          const UFace<Real> &uf = ut.face[f];
+          plane[q] = UPlane<Real>{{uf.n[0], uf.n[1], uf.n[2]}, uf.d};
+          link[q] = ULink<Real>{uf.nbr, uf.nbr >= 0 ? pstart[uf.nbr] : 0u, uf.nbr >= 0 ? pstart[uf.nbr + 1] : 0u,
+                                {uf.sh[0], uf.sh[1], uf.sh[2]}};
+          nbr[f] = uf.nbr;
+          const double ad = std::fabs(static_cast<double>(uf.d));
+          if (!(ad >= 0x1p-30 && ad <= 0x1p50)) u_tame = false;
+        }
+      upv(u_plane_start, pstart);
+      upv(u_face_nbr, nbr);
+      upv(u_plane, plane);
+      upv(u_link, link);
       upv(u_face_centroid, ut.face_centroid);
       std::vector<double2> geo(ut.face.size());
       for (size_t f = 0; f < geo.size(); ++f) geo[f] = make_double2(ut.face_geo[2 * f], ut.face_geo[2 * f + 1]);
@@ -712,23 +739,10 @@ struct Engine final : EngineBase {
       tal.pint_fp = nullptr;
       tal.esc_fp = nullptr;
     }
-    {
-      const size_t R1 = kTallyReplicas - 1;
-      tal.ncell = N;
-      rep_u32.ensure(R1 * N);
-      tal.segs_rep = rep_u32.p;
-      if (precision == STORM_GPU_FP64) {
-        rep_f64.ensure(R1 * 2 * static_cast<size_t>(N));
-        tal.dep_fp_rep = rep_f64.p;
-        tal.pint_fp_rep = rep_f64.p + R1 * N;
-        tal.dep_rep = tal.pint_rep = nullptr;
-      } else {
-        rep_u64.ensure(R1 * 2 * n2);
-        tal.dep_rep = rep_u64.p;
-        tal.pint_rep = rep_u64.p + R1 * n2;
-        tal.dep_fp_rep = tal.pint_fp_rep = nullptr;
-      }
-    }
+    tal.ncell = N;
+    tal.rec_words = cache_fields() == 1u ? 2u : 4u;
+    rec.ensure(static_cast<size_t>(kTallyReplicas) * N * tal.rec_words);
+    tal.rec = rec.p;
     // per-group time-averaged radiation energy (withEgTimeAvg, multigroup)
     eg_on = groups >= 2 && p->groups.with_eg_time_avg != 0;
     tal.eg = nullptr;
@@ -864,20 +878,23 @@ struct Engine final : EngineBase {
     for (int f = 0; f < 6; ++f)
       if (bnd.face_kind[f] == STORM_FACE_ESCAPE) m.escape_mask |= 1u << f;
     m.face_start = u_face_start.p;
-    m.face = u_face.p;
+    m.plane_start = u_plane_start.p;
+    m.tame = u_tame ? 1u : 0u;
+    m.plane = u_plane.p;
+    m.link = u_link.p;
     m.face_centroid = u_face_centroid.p;
     m.ddmc_rate = imc.with_ddmc ? u_ddmc_rate.p : nullptr;
     m.spec = spectrum();
     return m;
   }
   // Per transport kernel and block size: the blocks its registers let run
-  // on one CU, and the tally-cache slots (the share of the CU's LDS of each
+  // on one CU, and the tally-cache groups (the share of the CU's LDS of each
   // such block) for each chunking.
   static int chunk_index(int32_t k) { return k == 1 ? 0 : (k == 2 ? 1 : (k == 4 ? 2 : (k == 8 ? 3 : 4))); }
   static int block_index(int32_t b) { return b == 64 ? 0 : (b == 128 ? 1 : (b == 256 ? 2 : 3)); }
   struct KernelFit {
     uint32_t per_cu = 0;
-    uint32_t slots[5] = {};
+    uint32_t groups[5] = {};
   };
   KernelFit fit_cache[2][2][4][4];  // [refill][polyhedral][F][block]
   int n_cu = 0;
@@ -908,33 +925,38 @@ struct Engine final : EngineBase {
       ch >>= 1;
     return ch;
   }
-  uint32_t slots_of(KernelFit &f, int32_t ch, uint32_t nf) {
-    uint32_t &r = f.slots[chunk_index(ch)];
-    if (!r) r = cache_slots(static_cast<uint32_t>(block) * static_cast<uint32_t>(ch), nf, f.per_cu);
+  uint32_t groups_of(KernelFit &f, int32_t ch, uint32_t nf) {
+    uint32_t &r = f.groups[chunk_index(ch)];
+    if (!r)
+      r = cache_groups(static_cast<uint32_t>(block) * static_cast<uint32_t>(ch), nf, f.per_cu,
+                       static_cast<uint32_t>(block) / 64u);
     return r;
   }
+  // 64-bit sums per slot of the transport's tally table
+  uint32_t cache_fields() const { return (precision == STORM_GPU_MIXED && groups < 2) ? 1u : 2u; }
 
   // One transport launch on the kernel variant compiled for this problem's
   // features (random walk / DDMC, multigroup) and mesh, in the schedule in use.
   template <uint32_t F, typename MeshT>
   void launch_transport_m(uint64_t n_in, PacketBufs<Real> &src, PacketBufs<Real> &dst, const MeshT &mesh,
                           const AccelView<Real> &av, const StepConsts &kc) {
-    const uint32_t nf = (precision == STORM_GPU_MIXED && groups < 2) ? 1u : 2u;
+    const uint32_t nf = cache_fields();
     const bool refill = schedule == STORM_GPU_SCHEDULE_REFILL;
     KernelFit &f = refill ? fit_for(k_transport_refill<Real, F, MeshT>, true, F, block)
                           : fit_for(k_transport<Real, F, MeshT>, false, F, block);
     const int32_t ch = launch_chunks(f, n_in);
-    const uint32_t slots = slots_of(f, ch, nf);
+    const uint32_t ngroups = groups_of(f, ch, nf);
+    const uint32_t lds = cache_bytes(ngroups, nf, static_cast<uint32_t>(block) / 64u);
     const uint32_t chunks = static_cast<uint32_t>(ch) * static_cast<uint32_t>(block / 64);
     const uint32_t grid = blocks_for(n_in, 64u * chunks);
     if (refill) {
-      k_transport_refill<Real, F, MeshT><<<grid, block, cache_bytes(slots, nf), stream>>>(
+      k_transport_refill<Real, F, MeshT><<<grid, block, lds, stream>>>(
           static_cast<uint32_t>(n_in), src.soa(), dst.soa(), counters_u32.p, cpre.soa(), counters_u32.p + 1, mesh,
-          xs.p, av, kc, seg_per_pass, tal, leaving.p, slots, nf, chunks, cstage.soa());
+          xs.p, av, kc, seg_per_pass, tal, leaving.p, ngroups, nf, chunks, cstage.soa());
     } else {
-      k_transport<Real, F, MeshT><<<grid, block, cache_bytes(slots, nf), stream>>>(
+      k_transport<Real, F, MeshT><<<grid, block, lds, stream>>>(
           static_cast<uint32_t>(n_in), src.soa(), dst.soa(), counters_u32.p, cpre.soa(), counters_u32.p + 1, mesh,
-          xs.p, av, kc, seg_per_pass, tal, leaving.p, slots, nf, chunks);
+          xs.p, av, kc, seg_per_pass, tal, leaving.p, ngroups, nf, chunks);
     }
   }
   template <uint32_t F>
@@ -1031,12 +1053,10 @@ struct Engine final : EngineBase {
       ZeroBatch z;
       zero_add(z, tally_u64.p, tally_u64.n * sizeof(unsigned long long));
       if (precision == STORM_GPU_FP64) zero_add(z, tally_f64.p, tally_f64.n * sizeof(double));
-      zero_add(z, tal.segs, 2 * static_cast<size_t>(N) * sizeof(uint32_t));
+      zero_add(z, tal.begin, static_cast<size_t>(N) * sizeof(uint32_t));
       zero_add(z, tal.eg, static_cast<size_t>(N) * tal.eg_groups * sizeof(unsigned long long));
       zero_add(z, tal.eg_fp, static_cast<size_t>(N) * tal.eg_groups * sizeof(double));
-      zero_add(z, rep_u32.p, rep_u32.n * sizeof(uint32_t));
-      if (precision == STORM_GPU_FP64) zero_add(z, rep_f64.p, rep_f64.n * sizeof(double));
-      else zero_add(z, rep_u64.p, rep_u64.n * sizeof(unsigned long long));
+      zero_add(z, rec.p, static_cast<size_t>(kTallyReplicas) * N * tal.rec_words * sizeof(unsigned long long));
       zero_add(z, requant.p, requant.n * sizeof(unsigned long long));
       zero_add(z, leaving.p, 5 * sizeof(unsigned long long));
       zero_add(z, counters_u32.p, 2 * sizeof(uint32_t));
@@ -1056,7 +1076,7 @@ struct Engine final : EngineBase {
           sig_s_cell.p, fleck.p, sig_a.p, sig_s.p, Eemit.p, err.p, chord.p,
           imc.with_random_walk ? imc.rw_min_cell_optical_depth : HUGE_VAL, accel_on ? accel.p : nullptr,
           (imc.with_ddmc && imc.ddmc_multigroup_pgrw) ? imc.ddmc_min_cell_optical_depth : -1.0,
-          accel_on ? Dtil.p : nullptr);
+          accel_on ? Dtil.p : nullptr, accelview().rw_particle_tau);
     } else {
       k_prestep<Real><<<blocks_for(N, 256), 256, 0, stream>>>(
           N, T.p, md, have_host_sa ? host_sa.p : nullptr, have_host_ss ? host_ss.p : nullptr,
@@ -1066,10 +1086,10 @@ struct Engine final : EngineBase {
       k_accel_cells<Real><<<blocks_for(N, 256), 256, 0, stream>>>(
           N, chord.p, sig_a.p, sig_s.p, fleck.p, imc.with_random_walk, imc.rw_min_cell_optical_depth, imc.with_ddmc,
           imc.ddmc_min_cell_optical_depth, groups >= 2 ? 1 : 0, imc.ddmc_multigroup_pgrw ? 1 : 0, Dtil.p,
-          accel.p);
+          accel.p, xs.p, accelview().rw_particle_tau, accelview().ddmc_particle_tau);
       if (unstructured) {
         if (imc.with_ddmc)
-          k_accel_rates_u<Real><<<blocks_for(N, 256), 256, 0, stream>>>(N, u_face_start.p, u_face.p, u_face_geo.p, V.p,
+          k_accel_rates_u<Real><<<blocks_for(N, 256), 256, 0, stream>>>(N, u_face_start.p, u_face_nbr.p, u_face_geo.p, V.p,
                                                                          Dtil.p, accel.p, u_ddmc_rate.p);
       } else {
         k_accel_rates<Real><<<blocks_for(N, 256), 256, 0, stream>>>(N, d, meshview(), Dtil.p, accel.p);
@@ -1313,7 +1333,7 @@ struct Engine final : EngineBase {
       n_cen_total = h[1];
       ping = !ping;
     }
-    k_fold_replicas<<<blocks_for(N, 256), 256, 0, stream>>>(tal, kTallyReplicas, err.p);
+    k_fold_replicas<<<blocks_for(N, 256), 256, 0, stream>>>(tal, err.p);
     counters.seconds_transport = t_transport;
     counters.seconds_transport_max_launch = t_max;
     counters.census_before_comb = n_cen_total;

@@ -139,14 +139,18 @@ struct Tallies {
   double *esc_fp;            // [N]  FP64 engine: escaped
   uint32_t *segs;            // [N]  tracked segments (cellsStepsCounters)
   uint32_t *begin;           // [N]  packets per cell at transport start
-  // Replicas 1..kTallyReplicas-1 of the per-visit tallies (dep, pint, segs;
-  // dep_fp, pint_fp in the FP64 engine), one per XCD, each laid out as its
-  // replica-0 array above; k_fold_replicas adds them into replica 0 after
-  // the transport.  A wavefront adds into the replica of the XCD it runs on,
-  // so that the atomics of different XCDs never share a cache line.
-  unsigned long long *dep_rep, *pint_rep;  // [(R-1) * 2N]
-  double *dep_fp_rep, *pint_fp_rep;        // [(R-1) * N]
-  uint32_t *segs_rep;                      // [(R-1) * N]
+  // The per-visit tallies while the transport runs, one record of `rec_words`
+  // 64-bit words per cell and XCD, [replica][cell]: the deposit, the path
+  // integral (not with 2 words) and the segments, as integers in the mixed
+  // engine and doubles in the FP64 engine.  A wavefront adds into the replica
+  // of the XCD it runs on, so that the atomics of different XCDs never share
+  // a cache line; k_fold_replicas sums them into dep, pint and segs above.
+  // One record per cell because an atomic costs what the 64-byte line it
+  // goes to costs, however many of the wavefront's lanes add to that line:
+  // 24 G requests/s measured for one, two or eight lanes of 64 bits each
+  // (65536 cells at random), so a visit's words go out side by side.
+  unsigned long long *rec;
+  uint32_t rec_words;  // 2 or 4
   uint32_t ncell;
   // per-group path integral (withEgTimeAvg), [cell * eg_groups + g]: quanta
   // of 2^et in the mixed engine, FP64 in the FP64 engine (null: off)
@@ -318,7 +322,7 @@ __global__ __launch_bounds__(256) void k_prestep_mg(
     Real *__restrict__ cdf, Real *__restrict__ sig_s_cell, double *__restrict__ fleck,
     double *__restrict__ sig_a_out, double *__restrict__ sig_s_out, double *__restrict__ Eemit,
     uint32_t *__restrict__ err, const double *__restrict__ chord_c, double rw_cell_tau,
-    CellAccel<Real> *__restrict__ rw_out, double ddmc_pgrw_tau, double *__restrict__ Dtil) {
+    CellAccel<Real> *__restrict__ rw_out, double ddmc_pgrw_tau, double *__restrict__ Dtil, Real rw_tau) {
   uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= N) return;
   const double Tc = T[c];
@@ -426,6 +430,9 @@ __global__ __launch_bounds__(256) void k_prestep_mg(
       r.e_cut = static_cast<Real>(bounds[cut] / units::kev);
     }
     rw_out[c] = r;
+    // the walk's radius; k_accel_cells sets it again where DDMC is on
+    r.flags &= 1u;
+    xs[c].r_acc = accel_radius<Real>(r, rw_tau, Real(0));
   }
 }
 
@@ -731,45 +738,54 @@ __global__ __launch_bounds__(256) void k_boundary(uint32_t n_bc, uint32_t npc, c
 // cell finds no slot within kCacheProbes probes goes straight to device
 // memory.  Integer sums are exact in any order; the FP64 engine's sums
 // (doubles in v[0], v[1]) change only their order.
-// The table lives in dynamic LDS: `slots` (a power of two) slots of `nf`
+// The table lives in dynamic LDS: `groups` groups of four slots of `nf`
 // 64-bit sums, a tag and a segment count each.  nf = 1 in the mixed gray
 // engine (the deposit, in quanta; the path integral, tallied only in cells
 // without absorption, goes to device memory), 2 in the mixed multigroup
 // engine (deposit and path integral), 2 in the FP64 engine (deposit and
-// path integral as doubles).  The host sizes it to what a block's share of
-// the CU's 160 KB of LDS holds (cache_slots).
+// path integral as doubles).  Four cells in a row hash to one group, so that
+// the records of a group lie in one or two 64-byte lines and reach device
+// memory together when the table is written out.  Any number of groups will
+// do: the host takes what a block's share of the CU's 160 KB of LDS holds
+// (cache_groups; with a power of two a quarter to a half of it stayed empty).
+// Beside it every wavefront has room to lay out its 64 lanes' visits that
+// found no slot (DeviceSink::add_records).
 constexpr uint32_t kCacheProbes = 2;
-inline __host__ __device__ uint32_t cache_bytes(uint32_t slots, uint32_t nf) {
-  return slots * (8u * nf + 8u) + 16u;
+inline __host__ __device__ uint32_t cache_bytes(uint32_t groups, uint32_t nf, uint32_t waves) {
+  return waves * 64u * 8u * (nf + 1u) + 4u * groups * (8u * nf + 8u) + 16u;
 }
-// Largest power-of-two slot count within 4 per packet of the block's range
-// and the LDS share of one block when `blocks_per_cu` blocks are resident.
-inline uint32_t cache_slots(uint32_t packets, uint32_t nf, uint32_t blocks_per_cu) {
-  const uint32_t budget = (160u * 1024u) / (blocks_per_cu ? blocks_per_cu : 1u) - 64u;
-  uint32_t s = 1;
-  while (2 * s <= 4 * packets && cache_bytes(2 * s, nf) <= budget) s *= 2;
-  return s;
+// Most groups within one group per packet of the block's range and the LDS
+// share of one block when `blocks_per_cu` blocks are resident (LDS is handed
+// out in pieces of 1280 bytes).
+inline uint32_t cache_groups(uint32_t packets, uint32_t nf, uint32_t blocks_per_cu, uint32_t waves) {
+  const uint32_t share = (160u * 1024u) / (blocks_per_cu ? blocks_per_cu : 1u) / 1280u * 1280u;
+  const uint32_t fixed = cache_bytes(0u, nf, waves);
+  const uint32_t room = share > fixed ? (share - fixed) / (4u * (8u * nf + 8u)) : 1u;
+  return packets < room ? (packets ? packets : 1u) : (room ? room : 1u);
 }
 struct TallyCache {
-  uint32_t bits, mask, nf;
-  unsigned long long *v;  // v[f * slots + s], f < nf
-  uint32_t *tag;          // cell + 1; 0: free
+  uint32_t groups, nf;
+  unsigned long long *stage;  // per wavefront 64 entries of nf + 1 words
+  unsigned long long *v;      // v[f * 4 groups + s], f < nf
+  uint32_t *tag;              // cell + 1; 0: free
   uint32_t *segs;
   uint32_t *waves_done;
   uint32_t *next_chunk;   // k_transport's chunks handed out so far
   uint32_t *staged;       // k_transport_refill: census packets staged by the block
-  __device__ __forceinline__ unsigned long long &at(uint32_t f, uint32_t s) const { return v[f * (mask + 1u) + s]; }
+  __device__ __forceinline__ unsigned long long &at(uint32_t f, uint32_t s) const { return v[f * (4u * groups) + s]; }
 };
 
-// Lays the table out in `lds` (cache_bytes(slots, nf) bytes) and clears it;
-// the caller synchronises the block before first use.
-__device__ __forceinline__ TallyCache cache_init(unsigned char *lds, uint32_t slots, uint32_t nf) {
+// Lays the table out in `lds` (cache_bytes(groups, nf, waves) bytes) and
+// clears it; the caller synchronises the block before first use.
+__device__ __forceinline__ TallyCache cache_init(unsigned char *lds, uint32_t groups, uint32_t nf) {
   TallyCache L;
-  L.bits = 31u - static_cast<uint32_t>(__clz(static_cast<int>(slots)));
-  L.mask = slots - 1u;
+  const uint32_t slots = 4u * groups;
+  L.groups = groups;
   L.nf = nf;
-  L.v = reinterpret_cast<unsigned long long *>(lds);
-  L.tag = reinterpret_cast<uint32_t *>(lds + 8 * nf * slots);
+  unsigned long long *w = reinterpret_cast<unsigned long long *>(lds);
+  L.stage = w + (threadIdx.x >> 6) * 64u * (nf + 1u);
+  L.v = w + (blockDim.x >> 6) * 64u * (nf + 1u);
+  L.tag = reinterpret_cast<uint32_t *>(L.v + nf * slots);
   L.segs = L.tag + slots;
   L.waves_done = L.segs + slots;
   L.next_chunk = L.waves_done + 1;
@@ -794,94 +810,123 @@ __device__ __forceinline__ void lds_add(T *p, T v) {
 }
 
 // Slot of cell c (claimed if free), or -1 when the probed slots hold other cells.
-__device__ __forceinline__ int cache_slot(uint32_t *tag, uint32_t bits, uint32_t mask, uint32_t c) {
+__device__ __forceinline__ int cache_slot(const TallyCache &L, uint32_t c) {
   const uint32_t key = c + 1u;
-  const uint32_t h = (c * 0x9E3779B1u) >> (32u - bits);
+  uint32_t g = __umulhi((c >> 2) * 0x9E3779B1u, L.groups);
   int found = -1;
   for (uint32_t probe = 0; probe < kCacheProbes && found < 0; ++probe) {
-    const uint32_t s = (h + probe) & mask;
-    uint32_t cur = __hip_atomic_load(&tag[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    if (cur == 0u) cur = atomicCAS(&tag[s], 0u, key);
+    const uint32_t s = 4u * g + (c & 3u);
+    uint32_t cur = __hip_atomic_load(&L.tag[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    if (cur == 0u) cur = atomicCAS(&L.tag[s], 0u, key);
     if (cur == 0u || cur == key) found = static_cast<int>(s);
+    g = g + 1u < L.groups ? g + 1u : 0u;
   }
   return found;
 }
 
 struct DeviceSink {
-  Tallies t;
+  const Tallies &t;
   int32_t eq;
   uint32_t rw = 0, ddmc = 0;
-  // this wavefront's replica of the per-visit tallies
-  unsigned long long *dep, *pint;
-  double *dep_fp, *pint_fp;
-  uint32_t *segs;
-  TallyCache cache{};  // the block's LDS cache (cache.v null: none)
-  __device__ DeviceSink(const Tallies &tt, int32_t e) : t(tt), eq(e) {
-    // the integer replicas exist in the mixed engine, the FP64 ones in the
-    // FP64 engine (the other pair of pointers is null)
-    const uint32_t r = xcd_index() % kTallyReplicas;
-    const size_t n = tt.ncell;
-    dep = (r && tt.dep_rep) ? tt.dep_rep + (r - 1) * 2 * n : tt.dep;
-    pint = (r && tt.pint_rep) ? tt.pint_rep + (r - 1) * 2 * n : tt.pint;
-    segs = r ? tt.segs_rep + (r - 1) * n : tt.segs;
-    dep_fp = (r && tt.dep_fp_rep) ? tt.dep_fp_rep + (r - 1) * n : tt.dep_fp;
-    pint_fp = (r && tt.pint_fp_rep) ? tt.pint_fp_rep + (r - 1) * n : tt.pint_fp;
+  uint32_t rep;        // this wavefront's replica of the per-visit tallies
+  TallyCache cache;    // the block's LDS cache
+  __device__ DeviceSink(const Tallies &tt, int32_t e, const TallyCache &L)
+      : t(tt), eq(e), rep(xcd_index() % kTallyReplicas), cache(L) {}
+  __device__ unsigned long long *records() const {
+    return t.rec + static_cast<size_t>(rep) * t.ncell * t.rec_words;
   }
-  // Whole values (below 2^62 quanta, as is every sum of them) into the low
-  // word of the cell's pair: one atomic per tally.
+  // Visits that found no slot, straight into their cells' records: the lanes
+  // lay them out in the wavefront's part of LDS and then take one word of a
+  // visit each, so that a visit's words go out in one instruction and one
+  // 64-byte request instead of one each (u64 + u32 from two arrays 12.7 G
+  // visits/s, side by side 23.7).  T: how the words add.
+  template <typename T>
+  __device__ void add_records(bool miss, uint32_t c, unsigned long long a, unsigned long long b, uint32_t n) const {
+    const uint64_t mask = __builtin_amdgcn_ballot_w64(miss);
+    if (!mask) return;
+    const uint32_t nf = cache.nf, S = nf + 1u;
+    if (miss) {
+      unsigned long long *e = cache.stage + lane_rank(mask) * S;
+      e[0] = a;
+      if (nf >= 2u) e[1] = b;
+      e[nf] = (static_cast<unsigned long long>(c) << 32) | n;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const uint64_t active = __builtin_amdgcn_ballot_w64(true);
+    const uint32_t items = static_cast<uint32_t>(__popcll(mask)) * t.rec_words;
+    unsigned long long *rec = records();
+    for (uint32_t i = lane_rank(active); i < items; i += static_cast<uint32_t>(__popcll(active))) {
+      const uint32_t q = t.rec_words == 2u ? i >> 1 : i >> 2, word = i & (t.rec_words - 1u);
+      if (word > nf) continue;
+      const unsigned long long *e = cache.stage + q * S;
+      const unsigned long long last = e[nf];
+      put<T>(rec, static_cast<uint32_t>(last >> 32), word, e[word], static_cast<uint32_t>(last));
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+  // adds word `word` of a visit (bits: its value; n: its segments) to cell c
+  template <typename T>
+  __device__ void put(unsigned long long *rec, uint32_t c, uint32_t word, unsigned long long bits, uint32_t n) const {
+    T v;
+    if (word == cache.nf) v = static_cast<T>(n);
+    else __builtin_memcpy(&v, &bits, sizeof v);
+    if (v != T(0)) atomicAdd(reinterpret_cast<T *>(rec) + static_cast<size_t>(c) * t.rec_words + word, v);
+  }
+  // Whole values (below 2^62 quanta, as is every sum of them) into one word.
   __device__ void visit(uint32_t c, fx::Limbs d, fx::Limbs e, uint32_t n) {
     const unsigned long long dv = fx::value_of(d), ev = fx::value_of(e);
-    const int s = cache.v ? cache_slot(cache.tag, cache.bits, cache.mask, c) : -1;
+    const int s = cache_slot(cache, c);
     if (s >= 0) {
       if (dv) lds_add(&cache.at(0, s), dv);
-      if (cache.nf >= 2) {
-        if (ev) lds_add(&cache.at(1, s), ev);
-      } else if (ev) {
-        atomicAdd(&pint[2 * c], ev);
-      }
+      if (cache.nf >= 2 && ev) lds_add(&cache.at(1, s), ev);
       lds_add(&cache.segs[s], n);
-      return;
     }
-    if (dv) atomicAdd(&dep[2 * c], dv);
-    if (ev) atomicAdd(&pint[2 * c], ev);
-    atomicAdd(&segs[c], n);
+    if (cache.nf < 2 && ev) atomicAdd(&t.pint[2 * c], ev);
+    add_records<unsigned long long>(s < 0, c, dv, ev, n);
   }
   __device__ void roulette(uint32_t c, double w) { tally_limbs(t.rdep, c, fx::limbs_of(w, eq)); }
   __device__ void visit_fp(uint32_t c, double d, double e, uint32_t n) {
-    const int s = cache.v ? cache_slot(cache.tag, cache.bits, cache.mask, c) : -1;
+    const int s = cache_slot(cache, c);
     if (s >= 0) {
       if (d != 0.0) lds_add(reinterpret_cast<double *>(&cache.at(0, s)), d);
       if (e != 0.0) lds_add(reinterpret_cast<double *>(&cache.at(1, s)), e);
       lds_add(&cache.segs[s], n);
-      return;
     }
-    if (d != 0.0) atomicAdd(&dep_fp[c], d);
-    if (e != 0.0) atomicAdd(&pint_fp[c], e);
-    atomicAdd(&segs[c], n);
+    add_records<double>(s < 0, c, static_cast<unsigned long long>(__double_as_longlong(d)),
+                        static_cast<unsigned long long>(__double_as_longlong(e)), n);
   }
   // Called by every wavefront of the block once its packets are done: the
-  // last one writes the cache to device memory (and returns true).
+  // last one writes the cache to device memory (and returns true), a lane to
+  // each word, so that the records of four cells in a row go out together.
   __device__ bool finish_block() {
-    if (!cache.v) return false;
     uint32_t done = 0u;
     if (lane_rank(__builtin_amdgcn_ballot_w64(true)) == 0u)
       done = __hip_atomic_fetch_add(cache.waves_done, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
     done = __builtin_amdgcn_readfirstlane(done);
     if (done + 1u != (blockDim.x + 63u) / 64u) return false;
-    for (uint32_t s = __lane_id(); s <= cache.mask; s += 64u) {
-      const uint32_t key = __hip_atomic_load(&cache.tag[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-      if (!key) continue;
-      const uint32_t c = key - 1u;
-      if (dep_fp) {
-        const double d = __longlong_as_double(static_cast<long long>(cache.at(0, s)));
-        const double e = __longlong_as_double(static_cast<long long>(cache.at(1, s)));
-        if (d != 0.0) atomicAdd(&dep_fp[c], d);
-        if (e != 0.0) atomicAdd(&pint_fp[c], e);
-      } else {
-        if (cache.at(0, s)) atomicAdd(&dep[2 * c], cache.at(0, s));
-        if (cache.nf >= 2 && cache.at(1, s)) atomicAdd(&pint[2 * c], cache.at(1, s));
+    const uint32_t words = 4u * cache.groups * t.rec_words;
+    unsigned long long *rec = records();
+    // the keys of several rounds at a time, so that their reads overlap
+    constexpr uint32_t kRounds = 8;
+    for (uint32_t i0 = __lane_id(); i0 < words; i0 += 64u * kRounds) {
+      uint32_t key[kRounds];
+#pragma unroll
+      for (uint32_t j = 0; j < kRounds; ++j) {
+        const uint32_t i = i0 + 64u * j;
+        const uint32_t s = t.rec_words == 2u ? i >> 1 : i >> 2;
+        key[j] = i < words ? __hip_atomic_load(&cache.tag[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) : 0u;
       }
-      if (cache.segs[s]) atomicAdd(&segs[c], cache.segs[s]);
+#pragma unroll
+      for (uint32_t j = 0; j < kRounds; ++j) {
+        const uint32_t i = i0 + 64u * j;
+        const uint32_t s = t.rec_words == 2u ? i >> 1 : i >> 2, word = i & (t.rec_words - 1u);
+        if (!key[j] || word > cache.nf) continue;
+        const unsigned long long bits = word < cache.nf ? cache.at(word, s) : 0ull;
+        const uint32_t n = cache.segs[s];
+        if (t.dep_fp) put<double>(rec, key[j] - 1u, word, bits, n);
+        else put<unsigned long long>(rec, key[j] - 1u, word, bits, n);
+      }
     }
     return true;
   }
@@ -921,14 +966,13 @@ __device__ __forceinline__ void wave_add_u32(uint32_t v, unsigned long long *dst
   uint32_t n_in, PacketSoA<Real> in, PacketSoA<Real> out, uint32_t *__restrict__ n_out, CensusSoA<Real> cen,  \
       uint32_t *__restrict__ n_cen, MeshT mesh, const CellXS<Real> *__restrict__ xs,                          \
       AccelView<Real> acc, StepConsts k, int32_t max_segments, Tallies t,                                     \
-      unsigned long long *__restrict__ stats, uint32_t cache_slots, uint32_t cache_fields, uint32_t chunks
+      unsigned long long *__restrict__ stats, uint32_t cache_groups, uint32_t cache_fields, uint32_t chunks
 template <typename Real, uint32_t F, typename MeshT>
 __device__ __forceinline__ void transport_chunks(STORM_TRANSPORT_ARGS) {
   extern __shared__ __align__(16) unsigned char lds[];
-  const TallyCache cache = cache_init(lds, cache_slots, cache_fields);
+  const TallyCache cache = cache_init(lds, cache_groups, cache_fields);
   __syncthreads();
-  DeviceSink sink(t, k.eq);
-  sink.cache = cache;
+  DeviceSink sink(t, k.eq, cache);
   const uint32_t lane = __lane_id();
   const uint64_t base = static_cast<uint64_t>(blockIdx.x) * chunks * 64u;
   uint32_t escaped = 0, longest = 0;
@@ -964,25 +1008,17 @@ __device__ __forceinline__ void transport_chunks(STORM_TRANSPORT_ARGS) {
   }
 }
 
-// Waves per SIMD the history kernel is compiled for.  FP32: 6 (80 VGPRs, a
-// few dozen bytes of spill), measured 17% faster than the compiler's own
-// choice of 4 (98-118 VGPRs) on the 64^3 cube with the random walk and 5%
-// faster than 5 on the gray cube.  FP64: the compiler's choice (2-3 waves);
-// at 6 it spills 200-500 bytes per lane.
-template <typename Real>
+// Waves per SIMD the pass kernel is compiled for.
+template <typename Real, uint32_t F, typename MeshT>
 struct TransportWaves {
-  static constexpr int kMin = 1;
-};
-template <>
-struct TransportWaves<float> {
-  static constexpr int kMin = 6;
+  static constexpr int kMin = sizeof(Real) == 8 ? 1 : (F ? 4 : 5);
 };
 
 template <typename Real, uint32_t F, typename MeshT = MeshView<Real>>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(TransportWaves<Real>::kMin, 8))) void
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(TransportWaves<Real, F, MeshT>::kMin, 8))) void
 k_transport(STORM_TRANSPORT_ARGS) {
   transport_chunks<Real, F, MeshT>(n_in, in, out, n_out, cen, n_cen, mesh, xs, acc, k, max_segments, t, stats,
-                                   cache_slots, cache_fields, chunks);
+                                   cache_groups, cache_fields, chunks);
 }
 
 // Block-local lane refill (the refill schedule).  The block owns the same
@@ -1007,16 +1043,18 @@ constexpr uint32_t kRefillIdle = 4;
 template <typename Real, uint32_t F, typename MeshT>
 __device__ __forceinline__ void transport_refill(STORM_TRANSPORT_ARGS, CensusSoA<Real> stage) {
   extern __shared__ __align__(16) unsigned char lds[];
-  const TallyCache cache = cache_init(lds, cache_slots, cache_fields);
+  const TallyCache cache = cache_init(lds, cache_groups, cache_fields);
   __syncthreads();
-  DeviceSink sink(t, k.eq);
-  sink.cache = cache;
+  DeviceSink sink(t, k.eq, cache);
   const uint64_t base = static_cast<uint64_t>(blockIdx.x) * chunks * 64u;
   const uint64_t lim = base + static_cast<uint64_t>(chunks) * 64u < n_in ? base + static_cast<uint64_t>(chunks) * 64u
                                                                           : static_cast<uint64_t>(n_in);
   const uint32_t span = static_cast<uint32_t>(lim - base);  // packets of this block
   typename TrackerOf<Real, F, MeshT>::type tr;
-  bool busy = false;
+  // a lane's packet: in flight, ended (kCensus, kGone, kEscaped, or kPaused
+  // after `max_segments` segments) and not yet written back, or none
+  constexpr int kPaused = 4, kNone = 5;
+  int state = kNone;
   int32_t nseg = 0;
   // wave-uniform: the chunk being handed out, [pool_next, pool_end) of the
   // block's range, and whether the block's range is exhausted
@@ -1024,65 +1062,62 @@ __device__ __forceinline__ void transport_refill(STORM_TRANSPORT_ARGS, CensusSoA
   bool drained = false;
   uint32_t escaped = 0, longest = 0;
   for (;;) {
-    if (!drained) {
-      const uint64_t idle = __builtin_amdgcn_ballot_w64(!busy);
-      const uint32_t nidle = static_cast<uint32_t>(__popcll(idle));
-      if (nidle >= kRefillIdle) {
-        const uint32_t r = lane_rank(idle);
-        uint32_t given = 0;
-        while (given < nidle) {
-          if (pool_next >= pool_end) {
-            uint32_t ch = 0;
-            if (lane_rank(__builtin_amdgcn_ballot_w64(true)) == 0u)
-              ch = __hip_atomic_fetch_add(cache.next_chunk, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            ch = __builtin_amdgcn_readfirstlane(ch);
-            if (ch >= chunks || ch * 64u >= span) {
-              drained = true;
-              break;
-            }
-            pool_next = ch * 64u;
-            pool_end = pool_next + 64u < span ? pool_next + 64u : span;
-          }
-          const uint32_t avail = pool_end - pool_next;
-          const uint32_t take = nidle - given < avail ? nidle - given : avail;
-          if (!busy && r >= given && r < given + take) {
-            const Packet<Real> p = load_packet(in, static_cast<uint32_t>(base + pool_next + (r - given)));
-            tr.begin(p, mesh, xs, k);
-            busy = true;
-            nseg = 0;
-          }
-          pool_next += take;
-          given += take;
+    const uint64_t idle = __builtin_amdgcn_ballot_w64(state != kAlive);
+    const uint32_t nidle = static_cast<uint32_t>(__popcll(idle));
+    if (drained ? idle == ~0ull : nidle >= kRefillIdle) {
+      // write back the packets that ended
+      if (state != kAlive && state != kNone) {
+        Packet<Real> p;
+        p.flags = 0u;
+        tr.end(p, mesh, k, sink);
+        if (p.ctr > longest) longest = p.ctr;
+        escaped += state == kEscaped ? 1u : 0u;
+        const uint32_t oslot = wave_append(state == kPaused, n_out);
+        if (state == kPaused) store_packet(out, oslot, p);
+        const uint64_t want = __builtin_amdgcn_ballot_w64(state == kCensus);
+        if (want) {
+          uint32_t first = 0u;
+          if (lane_rank(__builtin_amdgcn_ballot_w64(true)) == 0u)
+            first = __hip_atomic_fetch_add(cache.staged, static_cast<uint32_t>(__popcll(want)), __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_WORKGROUP);
+          first = __builtin_amdgcn_readfirstlane(first);
+          if (state == kCensus) store_census(stage, static_cast<uint32_t>(base) + first + lane_rank(want), p);
         }
+        state = kNone;
       }
+      if (drained) break;
+      // and take the next ones of the block's range
+      const uint32_t rank = lane_rank(idle);
+      uint32_t given = 0;
+      while (given < nidle) {
+        if (pool_next >= pool_end) {
+          uint32_t ch = 0;
+          if (lane_rank(__builtin_amdgcn_ballot_w64(true)) == 0u)
+            ch = __hip_atomic_fetch_add(cache.next_chunk, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          ch = __builtin_amdgcn_readfirstlane(ch);
+          if (ch >= chunks || ch * 64u >= span) {
+            drained = true;
+            break;
+          }
+          pool_next = ch * 64u;
+          pool_end = pool_next + 64u < span ? pool_next + 64u : span;
+        }
+        const uint32_t avail = pool_end - pool_next;
+        const uint32_t take = nidle - given < avail ? nidle - given : avail;
+        if (state != kAlive && rank >= given && rank < given + take) {
+          const Packet<Real> p = load_packet(in, static_cast<uint32_t>(base + pool_next + (rank - given)));
+          tr.begin(p, mesh, xs, k);
+          state = kAlive;
+          nseg = 0;
+        }
+        pool_next += take;
+        given += take;
+      }
+      if (__builtin_amdgcn_ballot_w64(state == kAlive) == 0ull) break;  // the range was exhausted already
     }
-    // every lane idle: the block's range was exhausted on this or an earlier round
-    if (__builtin_amdgcn_ballot_w64(busy) == 0ull) break;
-    int outcome = kAlive;
-    if (busy) {
-      outcome = tr.segment(mesh, xs, acc, k, sink);
-      ++nseg;
-    }
-    const bool fin = busy && (outcome != kAlive || nseg >= max_segments);
-    Packet<Real> p;
-    if (fin) {
-      tr.end(p, k, sink);
-      busy = false;
-    }
-    const bool census = fin && outcome == kCensus;
-    const bool survivor = fin && outcome == kAlive;
-    escaped += (fin && outcome == kEscaped) ? 1u : 0u;
-    if (fin && p.ctr > longest) longest = p.ctr;
-    const uint32_t oslot = wave_append(survivor, n_out);
-    if (survivor) store_packet(out, oslot, p);
-    const uint64_t want = __builtin_amdgcn_ballot_w64(census);
-    if (want) {
-      uint32_t first = 0u;
-      if (lane_rank(__builtin_amdgcn_ballot_w64(true)) == 0u)
-        first = __hip_atomic_fetch_add(cache.staged, static_cast<uint32_t>(__popcll(want)), __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_WORKGROUP);
-      first = __builtin_amdgcn_readfirstlane(first);
-      if (census) store_census(stage, static_cast<uint32_t>(base) + first + lane_rank(want), p);
+    if (state == kAlive) {
+      state = tr.segment(mesh, xs, acc, k, sink);
+      if (++nseg >= max_segments && state == kAlive) state = kPaused;
     }
   }
   // the staged census becomes visible to the block's last wavefront
@@ -1103,25 +1138,17 @@ __device__ __forceinline__ void transport_refill(STORM_TRANSPORT_ARGS, CensusSoA
   }
 }
 
-// Waves per SIMD the refill kernel is compiled for.  FP32: 5 (96 VGPRs),
-// measured 17% faster than 6 on the cube (whose spills it reloads in its
-// per-segment loop: 77 B of HBM traffic per segment at 6) and 9% faster than
-// 4; on the step slab 4 and 5 are 8% and 5% faster than 6.  FP64: the
-// compiler's choice.
-template <typename Real>
+// Waves per SIMD the refill kernel is compiled for.
+template <typename Real, uint32_t F, typename MeshT>
 struct RefillWaves {
-  static constexpr int kMin = 1;
-};
-template <>
-struct RefillWaves<float> {
-  static constexpr int kMin = 5;
+  static constexpr int kMin = sizeof(Real) == 8 ? 1 : ((F & kFeatMultigroup) ? 4 : 5);
 };
 
 template <typename Real, uint32_t F, typename MeshT = MeshView<Real>>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RefillWaves<Real>::kMin, 8))) void
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RefillWaves<Real, F, MeshT>::kMin, 8))) void
 k_transport_refill(STORM_TRANSPORT_ARGS, CensusSoA<Real> stage) {
   transport_refill<Real, F, MeshT>(n_in, in, out, n_out, cen, n_cen, mesh, xs, acc, k, max_segments, t, stats,
-                                   cache_slots, cache_fields, chunks, stage);
+                                   cache_groups, cache_fields, chunks, stage);
 }
 #undef STORM_TRANSPORT_ARGS
 
@@ -1138,7 +1165,8 @@ __global__ __launch_bounds__(256) void k_accel_cells(uint32_t N, const double *_
                                                      const double *__restrict__ fleck, int32_t rw_on,
                                                      double rw_cell_tau, int32_t ddmc_on, double ddmc_cell_tau,
                                                      int32_t walk_set, int32_t ddmc_pgrw,
-                                                     double *__restrict__ Dtil, CellAccel<Real> *__restrict__ out) {
+                                                     double *__restrict__ Dtil, CellAccel<Real> *__restrict__ out,
+                                                     CellXS<Real> *__restrict__ xs, Real rw_tau, Real ddmc_tau) {
   uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= N) return;
   const double chord = chord_c[c];  // mean chord 4 V / S (RadiationIMC.hpp:1297-1298)
@@ -1165,6 +1193,7 @@ __global__ __launch_bounds__(256) void k_accel_cells(uint32_t N, const double *_
     // partial-gray DDMC data and D / c from k_prestep_mg (bit 2: eligible)
     if (ddmc_on && (pre & 4u)) a.flags |= 2u;
     out[c] = a;
+    xs[c].r_acc = accel_radius<Real>(a, rw_tau, ddmc_tau);
     return;
   }
   a.ddmc_sig_t = static_cast<Real>(st);
@@ -1174,6 +1203,9 @@ __global__ __launch_bounds__(256) void k_accel_cells(uint32_t N, const double *_
   Dtil[c] = Dt;
   if (ddmc_on && st * chord >= ddmc_cell_tau && Dt > 0.0) a.flags |= 2u;
   out[c] = a;
+  // (the rates may still clear the DDMC flag: the radius is then too small,
+  // which costs a look at the flags and no more)
+  xs[c].r_acc = accel_radius<Real>(a, rw_tau, ddmc_tau);
 }
 
 // Pass 2: leak rate per face, D_f A / (V d) / c with the harmonic mean of
@@ -1893,44 +1925,45 @@ __global__ __launch_bounds__(256) void k_zero_ranges(ZeroRanges r) {
   for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * 256u + threadIdx.x; i < n; i += stride) p[i] = 0u;
 }
 
-// Adds tally replicas 1..R-1 into replica 0, cell by cell in replica order
-// (integer sums are exact; the FP64 engine's sums are in a fixed order).
+// Sums the replicas of the per-visit tallies into dep, pint and segs, cell by
+// cell in replica order (integer sums are exact; the FP64 engine's sums are in
+// a fixed order); with 2-word records the transport has tallied pint itself.
 // Also the check of the two-limb tallies' bound: a cell's low limbs take up
 // to 2^28 additions of values below 2^36 within 64 bits, so a cell with 2^28
 // or more segments in the step sets kErrTallyOverflow here, before the comb
 // and postStep, and postStep then commits nothing.  The segment count
 // saturates at 2^32 - 1.
-__global__ __launch_bounds__(256) void k_fold_replicas(Tallies t, uint32_t reps, uint32_t *__restrict__ err) {
+template <typename T>
+__device__ __forceinline__ void fold_record(const Tallies &t, uint32_t c, T v[3]) {
+  const T *rec = reinterpret_cast<const T *>(t.rec);
+  v[0] = v[1] = v[2] = T(0);
+  for (uint32_t r = 0; r < kTallyReplicas; ++r) {
+    const T *e = rec + (static_cast<size_t>(r) * t.ncell + c) * t.rec_words;
+    v[0] += e[0];
+    if (t.rec_words == 4u) v[1] += e[1];
+    v[2] += e[t.rec_words == 4u ? 2 : 1];
+  }
+}
+__global__ __launch_bounds__(256) void k_fold_replicas(Tallies t, uint32_t *__restrict__ err) {
   const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= t.ncell) return;
-  const size_t n = t.ncell;
-  uint64_t sg = t.segs[c];
-  for (uint32_t r = 0; r + 1 < reps; ++r) sg += t.segs_rep[r * n + c];
+  uint64_t sg;
+  if (t.dep_fp) {
+    double v[3];
+    fold_record<double>(t, c, v);
+    t.dep_fp[c] = v[0];
+    t.pint_fp[c] = v[1];
+    sg = static_cast<uint64_t>(v[2]);
+  } else {
+    unsigned long long v[3];
+    fold_record<unsigned long long>(t, c, v);
+    t.dep[2 * c] = v[0];
+    t.dep[2 * c + 1] = 0ull;
+    if (t.rec_words == 4u) t.pint[2 * c] = v[1];
+    sg = v[2];
+  }
   t.segs[c] = sg > 0xFFFFFFFFull ? 0xFFFFFFFFu : static_cast<uint32_t>(sg);
   if (sg >= (1ull << 28)) atomicOr(err, kErrTallyOverflow);
-  if (t.dep_rep) {
-    unsigned long long d0 = t.dep[2 * c], d1 = t.dep[2 * c + 1];
-    unsigned long long p0 = t.pint[2 * c], p1 = t.pint[2 * c + 1];
-    for (uint32_t r = 0; r + 1 < reps; ++r) {
-      d0 += t.dep_rep[r * 2 * n + 2 * c];
-      d1 += t.dep_rep[r * 2 * n + 2 * c + 1];
-      p0 += t.pint_rep[r * 2 * n + 2 * c];
-      p1 += t.pint_rep[r * 2 * n + 2 * c + 1];
-    }
-    t.dep[2 * c] = d0;
-    t.dep[2 * c + 1] = d1;
-    t.pint[2 * c] = p0;
-    t.pint[2 * c + 1] = p1;
-  }
-  if (t.dep_fp_rep) {
-    double a = t.dep_fp[c], b = t.pint_fp[c];
-    for (uint32_t r = 0; r + 1 < reps; ++r) {
-      a += t.dep_fp_rep[r * n + c];
-      b += t.pint_fp_rep[r * n + c];
-    }
-    t.dep_fp[c] = a;
-    t.pint_fp[c] = b;
-  }
 }
 
 // Plain copy of n 16-byte words, one per thread: a kernel whose HBM traffic

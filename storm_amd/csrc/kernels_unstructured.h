@@ -165,7 +165,7 @@ __global__ __launch_bounds__(256) void k_boundary_u(uint32_t n_bc, uint32_t nsrc
 // (area, distance) per face.
 template <typename Real>
 __global__ __launch_bounds__(256) void k_accel_rates_u(uint32_t N, const uint32_t *__restrict__ face_start,
-                                                       const UFace<Real> *__restrict__ face,
+                                                       const int32_t *__restrict__ nbr,
                                                        const double2 *__restrict__ face_geo,
                                                        const double *__restrict__ V, const double *__restrict__ Dtil,
                                                        CellAccel<Real> *__restrict__ out, Real *__restrict__ rate) {
@@ -181,7 +181,7 @@ __global__ __launch_bounds__(256) void k_accel_rates_u(uint32_t N, const uint32_
   double total = 0.0;
   for (uint32_t f = f0; f < f1; ++f) {
     rate[f] = Real(0);
-    const int32_t nb = face[f].nbr;
+    const int32_t nb = nbr[f];
     if (nb < 0) continue;
     const double D2 = Dtil[nb];
     double Df = D1;
