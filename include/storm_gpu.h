@@ -292,6 +292,13 @@ int storm_gpu_debug_accel(storm_gpu_engine *eng, void *out, uint64_t *bytes);
 int storm_gpu_debug_spectrum(storm_gpu_engine *eng, int32_t *groups, double *nu_pow, void *bounds_kev, void *cdf,
                              void *sig_s);
 
+/* Checks the mixed engine's short arithmetic forms on the device: over the
+ * `count` floats whose bit patterns start at `first`, how many differ from
+ * the IEEE operation or the full function they stand for (op 0 reciprocal,
+ * 1 square root, 2 logarithm of a uniform, 3 e^x - 1 for x <= 0, 4 quotients
+ * of pairs made from the patterns).  No counterpart in the reference. */
+int storm_gpu_debug_math(int32_t op, uint32_t first, uint64_t count, uint64_t *mismatches);
+
 /* Measurement aid with no counterpart in the reference: one plain copy of
  * `bytes` (a multiple of 16) between two fresh device buffers by a kernel
  * that reads and writes each byte once (k_copy_calibration), so that a

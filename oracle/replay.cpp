@@ -325,7 +325,8 @@ void replay_philox(const uint32_t *ctr4, const uint32_t *key2, uint32_t *out4) {
 }
 
 // The engine's FP32 elementary functions on a batch (for accuracy tests):
-// which 0 log, 1 exp, 2 expm1, 3 sin(2 pi x), 4 cos(2 pi x).
+// which 0 log, 1 exp, 2 expm1, 3 sin(2 pi x), 4 cos(2 pi x), 5 log_unit,
+// 6 expm1_neg.
 void replay_fpmath(int32_t which, int64_t n, const float *x, float *y) {
   for (int64_t i = 0; i < n; ++i) {
     float s, c;
@@ -334,6 +335,8 @@ void replay_fpmath(int32_t which, int64_t n, const float *x, float *y) {
       case 1: y[i] = fpm::expf_d(x[i]); break;
       case 2: y[i] = fpm::expm1f_d(x[i]); break;
       case 3: fpm::sincos2pi(x[i], s, c); y[i] = s; break;
+      case 5: y[i] = fpm::log_unit(x[i]); break;
+      case 6: y[i] = fpm::expm1_neg(x[i]); break;
       default: fpm::sincos2pi(x[i], s, c); y[i] = c; break;
     }
   }

@@ -442,27 +442,23 @@ struct Engine final : EngineBase {
       nu_ref = p->groups.nu_ref;
       if (!(nu_ref > 0.0)) throw EngineError(1, "groups.nu_ref must be positive");
     }
-    // The starting schedule (the watch corrects it as the problem evolves),
-    // measured over the first steps at 256 threads: lanes refill from ranges
-    // of 8 chunks per wavefront (the 64^3 cube, steps 3-12: 25.8 against 18.0
-    // G segments/s for pass in the mixed engine, 13.5 against 8.2 in FP64;
-    // the step slab 19.2 against 16.4), 4 for the mixed engine on polyhedral
-    // meshes (the batch of slabs: 36.0 against 26.5); the mixed multigroup
-    // problem on a Voronoi mesh runs passes (10.9 against 9.8).
-    const bool mg_poly = unstructured && precision != STORM_GPU_FP64 && p->groups.num_groups >= 2;
-    schedule = mg_poly ? STORM_GPU_SCHEDULE_PASS : STORM_GPU_SCHEDULE_REFILL;
+    // The starting launch (the watch corrects the schedule as the problem
+    // evolves), measured in ms of transport per step: lanes refill, from ranges
+    // of 8 chunks per wavefront in 256-thread blocks (the 64^3 cube over 45
+    // steps: 6.1 against 6.7 from 4 and 8.0 from 16, whose cells no longer fit
+    // the LDS table; passes 11.5), of 4 in the mixed engine on polyhedral
+    // meshes (32 slabs in a batch 5.9 against 6.5 from 8; 64 groups on 3e4
+    // cells 4.9 against 4.9, passes 5.8).
+    schedule = STORM_GPU_SCHEDULE_REFILL;
     if (unstructured && precision != STORM_GPU_FP64) chunks_of[1] = 4;
-    // its passes from 1 chunk per wavefront (11.1 against 10.9 at 2)
-    if (mg_poly) chunks_of[0] = 1;
-    // the FP64 engine refills from 16 (its 2-3 waves per SIMD leave each
-    // block a larger LDS table): the cube as stated 15.4 against 14.9 G
-    // segments/s over 50 steps, the step slab even
+    if (unstructured && precision != STORM_GPU_FP64 && p->groups.num_groups >= 2) chunks_of[0] = 1;
+    // the FP64 engine from 16 (its 2-3 waves per SIMD leave each block a larger
+    // LDS table): the 64^3 cube 13.2 against 13.9 from 8
     if (precision == STORM_GPU_FP64) chunks_of[1] = 16;
-    // DDMC on a Cartesian mesh: 512-thread blocks refilling from 16 chunks
-    // per wavefront (the step slab, steps 3-8, mixed engine: 24.2 G
-    // segments/s against 19.3 at 256 threads and 8 chunks, 22.0 at 512 and 8,
-    // 18.7 at 256 and 16; FP64: 14.5 against 12.7)
-    if (!unstructured && imc.with_ddmc) {
+    // the mixed engine with DDMC on a Cartesian mesh from 16 in 512-thread
+    // blocks (the step slab over 45 steps: 11.8, in 256-thread blocks of 8 12.4;
+    // a launch of few rounds takes 8, launch_chunks)
+    if (!unstructured && imc.with_ddmc && precision != STORM_GPU_FP64) {
       block = 512;
       chunks_of[1] = 16;
     }
@@ -740,7 +736,7 @@ struct Engine final : EngineBase {
       tal.esc_fp = nullptr;
     }
     tal.ncell = N;
-    tal.rec_words = cache_fields() == 1u ? 2u : 4u;
+    tal.rec_words = (precision == STORM_GPU_MIXED && groups < 2) ? TallyFields<Real, 0u>::words : 4u;  // TallyFields
     rec.ensure(static_cast<size_t>(kTallyReplicas) * N * tal.rec_words);
     tal.rec = rec.p;
     // per-group time-averaged radiation energy (withEgTimeAvg, multigroup)
@@ -917,12 +913,19 @@ struct Engine final : EngineBase {
   // The chunks per wavefront of a launch over n_in packets: the schedule's,
   // halved while the launch would have fewer blocks than the device holds at
   // once (a small step in large block ranges leaves CUs idle: the 100-cell
-  // slab ran 5 times slower in ranges of 8 chunks).
+  // slab ran 5 times slower in ranges of 8 chunks), and from 16 to 8 already
+  // while it would be less than two and a half rounds of them, since the last
+  // round is then mostly empty (9.3e6 packets of the step slab in 512-thread
+  // blocks of 16 chunks, 2.2 rounds: 7.9 ms a launch, of 8 chunks 6.2; 3.7e6
+  // of the 32^3 cube in FP64, 1.8 and 3.6 rounds: 3.9 and 3.7).  Ranges of 8
+  // and less are not cut for that: 2e6 packets of the 30-group slab take 4.0
+  // ms in ranges of 4 chunks and 5.9 in ranges of 2.
   int32_t launch_chunks(const KernelFit &f, uint64_t n_in) const {
     int32_t ch = chunks_per_wave();
     const uint64_t resident = static_cast<uint64_t>(f.per_cu) * static_cast<uint64_t>(n_cu);
-    while (ch > 1 && (n_in + static_cast<uint64_t>(block) * ch - 1) / (static_cast<uint64_t>(block) * ch) < resident)
-      ch >>= 1;
+    auto blocks = [&](int32_t k) { return (n_in + static_cast<uint64_t>(block) * k - 1) / (static_cast<uint64_t>(block) * k); };
+    if (ch > 8 && 2 * blocks(ch) < 5 * resident) ch = 8;
+    while (ch > 1 && blocks(ch) < resident) ch >>= 1;
     return ch;
   }
   uint32_t groups_of(KernelFit &f, int32_t ch, uint32_t nf) {
@@ -932,15 +935,13 @@ struct Engine final : EngineBase {
                        static_cast<uint32_t>(block) / 64u);
     return r;
   }
-  // 64-bit sums per slot of the transport's tally table
-  uint32_t cache_fields() const { return (precision == STORM_GPU_MIXED && groups < 2) ? 1u : 2u; }
 
   // One transport launch on the kernel variant compiled for this problem's
   // features (random walk / DDMC, multigroup) and mesh, in the schedule in use.
   template <uint32_t F, typename MeshT>
   void launch_transport_m(uint64_t n_in, PacketBufs<Real> &src, PacketBufs<Real> &dst, const MeshT &mesh,
                           const AccelView<Real> &av, const StepConsts &kc) {
-    const uint32_t nf = cache_fields();
+    constexpr uint32_t nf = TallyFields<Real, F>::nf;
     const bool refill = schedule == STORM_GPU_SCHEDULE_REFILL;
     KernelFit &f = refill ? fit_for(k_transport_refill<Real, F, MeshT>, true, F, block)
                           : fit_for(k_transport<Real, F, MeshT>, false, F, block);
@@ -949,15 +950,25 @@ struct Engine final : EngineBase {
     const uint32_t lds = cache_bytes(ngroups, nf, static_cast<uint32_t>(block) / 64u);
     const uint32_t chunks = static_cast<uint32_t>(ch) * static_cast<uint32_t>(block / 64);
     const uint32_t grid = blocks_for(n_in, 64u * chunks);
-    if (refill) {
-      k_transport_refill<Real, F, MeshT><<<grid, block, lds, stream>>>(
-          static_cast<uint32_t>(n_in), src.soa(), dst.soa(), counters_u32.p, cpre.soa(), counters_u32.p + 1, mesh,
-          xs.p, av, kc, seg_per_pass, tal, leaving.p, ngroups, nf, chunks, cstage.soa());
-    } else {
-      k_transport<Real, F, MeshT><<<grid, block, lds, stream>>>(
-          static_cast<uint32_t>(n_in), src.soa(), dst.soa(), counters_u32.p, cpre.soa(), counters_u32.p + 1, mesh,
-          xs.p, av, kc, seg_per_pass, tal, leaving.p, ngroups, nf, chunks);
-    }
+    TransportArgs<Real, MeshT> a;
+    a.n_in = static_cast<uint32_t>(n_in);
+    a.chunks = chunks;
+    a.cache_groups = ngroups;
+    a.max_segments = seg_per_pass;
+    a.in = src.soa();
+    a.out = dst.soa();
+    a.n_out = counters_u32.p;
+    a.n_cen = counters_u32.p + 1;
+    a.cen = cpre.soa();
+    a.stage = cstage.soa();
+    a.mesh = mesh;
+    a.xs = xs.p;
+    a.acc = av;
+    a.k = kc;
+    a.t = tal;
+    a.stats = leaving.p;
+    if (refill) k_transport_refill<Real, F, MeshT><<<grid, block, lds, stream>>>(a);
+    else k_transport<Real, F, MeshT><<<grid, block, lds, stream>>>(a);
   }
   template <uint32_t F>
   void launch_transport_f(uint64_t n_in, PacketBufs<Real> &src, PacketBufs<Real> &dst, const MeshView<Real> &mv,
@@ -2042,6 +2053,20 @@ int storm_gpu_device_info(char *buf, size_t len) {
     HIPCHECK(hipGetDeviceProperties(&prop, dev));
     std::snprintf(buf, len, "%s | %s | CUs=%d | clock=%d kHz | mem=%zu MiB", prop.name, prop.gcnArchName,
                   prop.multiProcessorCount, prop.clockRate, static_cast<size_t>(prop.totalGlobalMem >> 20));
+  });
+}
+
+int storm_gpu_debug_math(int32_t op, uint32_t first, uint64_t count, uint64_t *mismatches) {
+  return guarded([&] {
+    if (op < 0 || op > 4 || !mismatches) throw EngineError(1, "op must be 0 .. 4 and mismatches given");
+    if (count > (1ull << 32)) throw EngineError(1, "at most 2^32 bit patterns");
+    DevBuf<unsigned long long> bad;
+    bad.ensure(1);
+    k_fill_u64<<<1, 64>>>(bad.p, 1, 0ull);
+    if (count) k_check_math<<<4096, 256>>>(op, first, count, bad.p);
+    unsigned long long h = 0;
+    HIPCHECK(hipMemcpy(&h, bad.p, sizeof h, hipMemcpyDeviceToHost));
+    *mismatches = h;
   });
 }
 

@@ -763,8 +763,10 @@ inline uint32_t cache_groups(uint32_t packets, uint32_t nf, uint32_t blocks_per_
   const uint32_t room = share > fixed ? (share - fixed) / (4u * (8u * nf + 8u)) : 1u;
   return packets < room ? (packets ? packets : 1u) : (room ? room : 1u);
 }
+template <uint32_t NF>
 struct TallyCache {
-  uint32_t groups, nf;
+  static constexpr uint32_t nf = NF;
+  uint32_t groups;
   unsigned long long *stage;  // per wavefront 64 entries of nf + 1 words
   unsigned long long *v;      // v[f * 4 groups + s], f < nf
   uint32_t *tag;              // cell + 1; 0: free
@@ -777,11 +779,11 @@ struct TallyCache {
 
 // Lays the table out in `lds` (cache_bytes(groups, nf, waves) bytes) and
 // clears it; the caller synchronises the block before first use.
-__device__ __forceinline__ TallyCache cache_init(unsigned char *lds, uint32_t groups, uint32_t nf) {
-  TallyCache L;
+template <uint32_t nf>
+__device__ __forceinline__ TallyCache<nf> cache_init(unsigned char *lds, uint32_t groups) {
+  TallyCache<nf> L;
   const uint32_t slots = 4u * groups;
   L.groups = groups;
-  L.nf = nf;
   unsigned long long *w = reinterpret_cast<unsigned long long *>(lds);
   L.stage = w + (threadIdx.x >> 6) * 64u * (nf + 1u);
   L.v = w + (blockDim.x >> 6) * 64u * (nf + 1u);
@@ -810,7 +812,8 @@ __device__ __forceinline__ void lds_add(T *p, T v) {
 }
 
 // Slot of cell c (claimed if free), or -1 when the probed slots hold other cells.
-__device__ __forceinline__ int cache_slot(const TallyCache &L, uint32_t c) {
+template <uint32_t nf>
+__device__ __forceinline__ int cache_slot(const TallyCache<nf> &L, uint32_t c) {
   const uint32_t key = c + 1u;
   uint32_t g = __umulhi((c >> 2) * 0x9E3779B1u, L.groups);
   int found = -1;
@@ -824,16 +827,57 @@ __device__ __forceinline__ int cache_slot(const TallyCache &L, uint32_t c) {
   return found;
 }
 
+// 64-bit sums per slot of the transport's tally table, and words of a record
+// (Tallies::rec): the mixed gray engine tallies no path integral there.
+template <typename Real, uint32_t F>
+struct TallyFields {
+  static constexpr uint32_t nf = (sizeof(Real) == 4 && (F & kFeatMultigroup) == 0u) ? 1u : 2u;
+  static constexpr uint32_t words = nf == 1u ? 2u : 4u;
+};
+
+// A transport kernel's arguments, its one parameter.
+// stats: [0] escapes, [1] random-walk steps, [2] DDMC steps, [4] longest history
+template <typename Real, typename MeshT>
+struct TransportArgs {
+  uint32_t n_in, chunks, cache_groups;
+  int32_t max_segments;
+  PacketSoA<Real> in, out;
+  uint32_t *n_out, *n_cen;
+  CensusSoA<Real> cen;
+  CensusSoA<Real> stage;  // refill: census staged per block
+  MeshT mesh;
+  const CellXS<Real> *xs;
+  AccelView<Real> acc;
+  StepConsts k;
+  Tallies t;
+  unsigned long long *stats;
+};
+// The arguments as they lie in the kernel's argument segment, for what is
+// used now and then (packet buffers, tallies, counters).  The compiler reads
+// every argument once at the kernel's start and keeps it in scalar registers,
+// of which there are 102; these arguments are more, so that it parked 40 to 70
+// of them in vector registers and fetched them back lane by lane inside the
+// segment loop (183 v_readlane in the random-walk kernel).  Behind the empty
+// asm the address is new to it at every use and they are read there.
+template <typename Args>
+__device__ __forceinline__ const Args &args_at_use() {
+  auto p = __builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const Args *)p;
+}
+
+template <typename Real, uint32_t F, typename MeshT>
 struct DeviceSink {
-  const Tallies &t;
+  using Args = TransportArgs<Real, MeshT>;
+  static constexpr uint32_t nf = TallyFields<Real, F>::nf, words = TallyFields<Real, F>::words;
   int32_t eq;
   uint32_t rw = 0, ddmc = 0;
-  uint32_t rep;        // this wavefront's replica of the per-visit tallies
-  TallyCache cache;    // the block's LDS cache
-  __device__ DeviceSink(const Tallies &tt, int32_t e, const TallyCache &L)
-      : t(tt), eq(e), rep(xcd_index() % kTallyReplicas), cache(L) {}
-  __device__ unsigned long long *records() const {
-    return t.rec + static_cast<size_t>(rep) * t.ncell * t.rec_words;
+  TallyCache<nf> cache;  // the block's LDS cache
+  __device__ DeviceSink(int32_t e, const TallyCache<nf> &L) : eq(e), cache(L) {}
+  // the records of this wavefront's XCD
+  __device__ static unsigned long long *records() {
+    const Tallies &t = args_at_use<Args>().t;
+    return t.rec + static_cast<size_t>(xcd_index() % kTallyReplicas) * t.ncell * words;
   }
   // Visits that found no slot, straight into their cells' records: the lanes
   // lay them out in the wavefront's part of LDS and then take one word of a
@@ -844,7 +888,7 @@ struct DeviceSink {
   __device__ void add_records(bool miss, uint32_t c, unsigned long long a, unsigned long long b, uint32_t n) const {
     const uint64_t mask = __builtin_amdgcn_ballot_w64(miss);
     if (!mask) return;
-    const uint32_t nf = cache.nf, S = nf + 1u;
+    constexpr uint32_t S = nf + 1u;
     if (miss) {
       unsigned long long *e = cache.stage + lane_rank(mask) * S;
       e[0] = a;
@@ -854,10 +898,10 @@ struct DeviceSink {
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
     const uint64_t active = __builtin_amdgcn_ballot_w64(true);
-    const uint32_t items = static_cast<uint32_t>(__popcll(mask)) * t.rec_words;
+    const uint32_t items = static_cast<uint32_t>(__popcll(mask)) * words;
     unsigned long long *rec = records();
     for (uint32_t i = lane_rank(active); i < items; i += static_cast<uint32_t>(__popcll(active))) {
-      const uint32_t q = t.rec_words == 2u ? i >> 1 : i >> 2, word = i & (t.rec_words - 1u);
+      const uint32_t q = i / words, word = i % words;
       if (word > nf) continue;
       const unsigned long long *e = cache.stage + q * S;
       const unsigned long long last = e[nf];
@@ -867,11 +911,11 @@ struct DeviceSink {
   }
   // adds word `word` of a visit (bits: its value; n: its segments) to cell c
   template <typename T>
-  __device__ void put(unsigned long long *rec, uint32_t c, uint32_t word, unsigned long long bits, uint32_t n) const {
+  __device__ static void put(unsigned long long *rec, uint32_t c, uint32_t word, unsigned long long bits, uint32_t n) {
     T v;
-    if (word == cache.nf) v = static_cast<T>(n);
+    if (word == nf) v = static_cast<T>(n);
     else __builtin_memcpy(&v, &bits, sizeof v);
-    if (v != T(0)) atomicAdd(reinterpret_cast<T *>(rec) + static_cast<size_t>(c) * t.rec_words + word, v);
+    if (v != T(0)) atomicAdd(reinterpret_cast<T *>(rec) + static_cast<size_t>(c) * words + word, v);
   }
   // Whole values (below 2^62 quanta, as is every sum of them) into one word.
   __device__ void visit(uint32_t c, fx::Limbs d, fx::Limbs e, uint32_t n) {
@@ -879,13 +923,13 @@ struct DeviceSink {
     const int s = cache_slot(cache, c);
     if (s >= 0) {
       if (dv) lds_add(&cache.at(0, s), dv);
-      if (cache.nf >= 2 && ev) lds_add(&cache.at(1, s), ev);
+      if (nf >= 2 && ev) lds_add(&cache.at(1, s), ev);
       lds_add(&cache.segs[s], n);
     }
-    if (cache.nf < 2 && ev) atomicAdd(&t.pint[2 * c], ev);
+    if (nf < 2 && ev) atomicAdd(&args_at_use<Args>().t.pint[2 * c], ev);
     add_records<unsigned long long>(s < 0, c, dv, ev, n);
   }
-  __device__ void roulette(uint32_t c, double w) { tally_limbs(t.rdep, c, fx::limbs_of(w, eq)); }
+  __device__ void roulette(uint32_t c, double w) { tally_limbs(args_at_use<Args>().t.rdep, c, fx::limbs_of(w, eq)); }
   __device__ void visit_fp(uint32_t c, double d, double e, uint32_t n) {
     const int s = cache_slot(cache, c);
     if (s >= 0) {
@@ -905,39 +949,40 @@ struct DeviceSink {
       done = __hip_atomic_fetch_add(cache.waves_done, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
     done = __builtin_amdgcn_readfirstlane(done);
     if (done + 1u != (blockDim.x + 63u) / 64u) return false;
-    const uint32_t words = 4u * cache.groups * t.rec_words;
+    const uint32_t all = 4u * cache.groups * words;
     unsigned long long *rec = records();
     // the keys of several rounds at a time, so that their reads overlap
     constexpr uint32_t kRounds = 8;
-    for (uint32_t i0 = __lane_id(); i0 < words; i0 += 64u * kRounds) {
+    for (uint32_t i0 = __lane_id(); i0 < all; i0 += 64u * kRounds) {
       uint32_t key[kRounds];
 #pragma unroll
       for (uint32_t j = 0; j < kRounds; ++j) {
         const uint32_t i = i0 + 64u * j;
-        const uint32_t s = t.rec_words == 2u ? i >> 1 : i >> 2;
-        key[j] = i < words ? __hip_atomic_load(&cache.tag[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) : 0u;
+        const uint32_t s = i / words;
+        key[j] = i < all ? __hip_atomic_load(&cache.tag[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) : 0u;
       }
 #pragma unroll
       for (uint32_t j = 0; j < kRounds; ++j) {
         const uint32_t i = i0 + 64u * j;
-        const uint32_t s = t.rec_words == 2u ? i >> 1 : i >> 2, word = i & (t.rec_words - 1u);
-        if (!key[j] || word > cache.nf) continue;
-        const unsigned long long bits = word < cache.nf ? cache.at(word, s) : 0ull;
+        const uint32_t s = i / words, word = i % words;
+        if (!key[j] || word > nf) continue;
+        const unsigned long long bits = word < nf ? cache.at(word, s) : 0ull;
         const uint32_t n = cache.segs[s];
-        if (t.dep_fp) put<double>(rec, key[j] - 1u, word, bits, n);
+        if (sizeof(Real) == 8) put<double>(rec, key[j] - 1u, word, bits, n);
         else put<unsigned long long>(rec, key[j] - 1u, word, bits, n);
       }
     }
     return true;
   }
   // escaped weight: in quanta (mixed engine) or as a double (FP64 engine)
-  __device__ void escape_fx(uint32_t c, double w) { tally_limbs(t.esc, c, fx::limbs_of(w, eq)); }
-  __device__ void escape_fp(uint32_t c, double w) { atomicAdd(&t.esc_fp[c], w); }
+  __device__ void escape_fx(uint32_t c, double w) { tally_limbs(args_at_use<Args>().t.esc, c, fx::limbs_of(w, eq)); }
+  __device__ void escape_fp(uint32_t c, double w) { atomicAdd(&args_at_use<Args>().t.esc_fp[c], w); }
   __device__ void rw_step() { ++rw; }
   __device__ void ddmc_step() { ++ddmc; }
   // path integral v (erg cm) of cell c in group g: rounded without bias to
   // the path-integral quantum in the mixed engine (u24: the draw)
   __device__ void group_path(uint32_t c, int32_t g, double v, const StepConsts &k, uint32_t u24) {
+    const Tallies &t = args_at_use<Args>().t;
     const size_t i = static_cast<size_t>(c) * t.eg_groups + static_cast<uint32_t>(g);
     if (t.eg_fp) {
       atomicAdd(&t.eg_fp[i], v);
@@ -961,18 +1006,14 @@ __device__ __forceinline__ void wave_add_u32(uint32_t v, unsigned long long *dst
 // chunk.  The packets come ordered by cell, so the block's range is a compact
 // region and its LDS tally table serves all of it; each cell it touched is
 // written to device memory once, when the block's last wavefront ends.
-// stats: [0] escapes, [1] random-walk steps, [2] DDMC steps, [4] longest history
-#define STORM_TRANSPORT_ARGS                                                                                  \
-  uint32_t n_in, PacketSoA<Real> in, PacketSoA<Real> out, uint32_t *__restrict__ n_out, CensusSoA<Real> cen,  \
-      uint32_t *__restrict__ n_cen, MeshT mesh, const CellXS<Real> *__restrict__ xs,                          \
-      AccelView<Real> acc, StepConsts k, int32_t max_segments, Tallies t,                                     \
-      unsigned long long *__restrict__ stats, uint32_t cache_groups, uint32_t cache_fields, uint32_t chunks
 template <typename Real, uint32_t F, typename MeshT>
-__device__ __forceinline__ void transport_chunks(STORM_TRANSPORT_ARGS) {
+__device__ __forceinline__ void transport_chunks(const TransportArgs<Real, MeshT> &a) {
+  using Args = TransportArgs<Real, MeshT>;
   extern __shared__ __align__(16) unsigned char lds[];
-  const TallyCache cache = cache_init(lds, cache_groups, cache_fields);
+  const auto cache = cache_init<TallyFields<Real, F>::nf>(lds, a.cache_groups);
   __syncthreads();
-  DeviceSink sink(t, k.eq, cache);
+  DeviceSink<Real, F, MeshT> sink(a.k.eq, cache);
+  const uint32_t chunks = a.chunks, n_in = a.n_in;
   const uint32_t lane = __lane_id();
   const uint64_t base = static_cast<uint64_t>(blockIdx.x) * chunks * 64u;
   uint32_t escaped = 0, longest = 0;
@@ -986,29 +1027,36 @@ __device__ __forceinline__ void transport_chunks(STORM_TRANSPORT_ARGS) {
     int outcome = kGone;
     Packet<Real> p;
     if (valid) {
-      p = load_packet(in, static_cast<uint32_t>(i));
-      outcome = transport_packet<Real, F>(p, mesh, xs, acc, k, max_segments, sink);
+      p = load_packet(args_at_use<Args>().in, static_cast<uint32_t>(i));
+      outcome = transport_packet<Real, F>(p, a.mesh, a.xs, a.acc, a.k, a.max_segments, sink);
     }
     const bool alive = valid && outcome == kAlive;
     const bool census = valid && outcome == kCensus;
-    uint32_t slot = wave_append(alive, n_out);
-    if (alive) store_packet(out, slot, p);
-    uint32_t cslot = wave_append(census, n_cen);
-    if (census) store_census(cen, cslot, p);
+    const Args &q = args_at_use<Args>();
+    uint32_t slot = wave_append(alive, q.n_out);
+    if (alive) store_packet(q.out, slot, p);
+    uint32_t cslot = wave_append(census, q.n_cen);
+    if (census) store_census(q.cen, cslot, p);
     escaped += (valid && outcome == kEscaped) ? 1u : 0u;
     if (valid && p.ctr > longest) longest = p.ctr;
     if (base + static_cast<uint64_t>(ch + 1u) * 64u >= n_in) break;  // the last chunk of the input
   }
   sink.finish_block();
+  unsigned long long *stats = args_at_use<Args>().stats;
   wave_add_u32(escaped, &stats[0]);
   wave_max_u32(longest, &stats[4]);
-  if (acc.cell) {
+  if ((F & kFeatAccel) != 0u) {
     wave_add_u32(sink.rw, &stats[1]);
     wave_add_u32(sink.ddmc, &stats[2]);
   }
 }
 
-// Waves per SIMD the pass kernel is compiled for.
+// Waves per SIMD the pass kernel is compiled for: in FP32 the most that leave
+// it without spills (80-96 VGPRs at 5, up to 124 at 4).  A spill is more than
+// its traffic: this compiler stores some before the wavefront's lanes are all
+// switched on again at the end of a branch, and a value that the other lanes
+// still need is then lost (seen in the escape and walk counters of a build
+// that spilled 100 bytes).  FP64: the compiler's choice (2-3 waves).
 template <typename Real, uint32_t F, typename MeshT>
 struct TransportWaves {
   static constexpr int kMin = sizeof(Real) == 8 ? 1 : (F ? 4 : 5);
@@ -1016,9 +1064,8 @@ struct TransportWaves {
 
 template <typename Real, uint32_t F, typename MeshT = MeshView<Real>>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(TransportWaves<Real, F, MeshT>::kMin, 8))) void
-k_transport(STORM_TRANSPORT_ARGS) {
-  transport_chunks<Real, F, MeshT>(n_in, in, out, n_out, cen, n_cen, mesh, xs, acc, k, max_segments, t, stats,
-                                   cache_groups, cache_fields, chunks);
+k_transport(TransportArgs<Real, MeshT> a) {
+  transport_chunks<Real, F, MeshT>(a);
 }
 
 // Block-local lane refill (the refill schedule).  The block owns the same
@@ -1037,15 +1084,20 @@ k_transport(STORM_TRANSPORT_ARGS) {
 // copies them there.  Appending them one or two at a time as lanes finish
 // would put an atomic per census packet on the one census counter that every
 // wavefront of the launch shares.
-// Idle lanes that take new packets together: 2, 4 and 16 measured within 1%
-// of each other (cube, step slab, batch of slabs).
-constexpr uint32_t kRefillIdle = 4;
+// Lanes whose packets ended are written back and given new ones 8 at a time,
+// so that the wavefront runs that code (some 250 instructions and two memory
+// round trips, for however few lanes) once in a while: against 4 at a time the
+// 64^3 cube takes 5.9 against 6.0 ms, the FP64 cube 3.77 against 3.88; 16 at a
+// time is even with 8.
+constexpr uint32_t kRefillIdle = 8;
 template <typename Real, uint32_t F, typename MeshT>
-__device__ __forceinline__ void transport_refill(STORM_TRANSPORT_ARGS, CensusSoA<Real> stage) {
+__device__ __forceinline__ void transport_refill(const TransportArgs<Real, MeshT> &a) {
+  using Args = TransportArgs<Real, MeshT>;
   extern __shared__ __align__(16) unsigned char lds[];
-  const TallyCache cache = cache_init(lds, cache_groups, cache_fields);
+  const auto cache = cache_init<TallyFields<Real, F>::nf>(lds, a.cache_groups);
   __syncthreads();
-  DeviceSink sink(t, k.eq, cache);
+  DeviceSink<Real, F, MeshT> sink(a.k.eq, cache);
+  const uint32_t chunks = a.chunks, n_in = a.n_in;
   const uint64_t base = static_cast<uint64_t>(blockIdx.x) * chunks * 64u;
   const uint64_t lim = base + static_cast<uint64_t>(chunks) * 64u < n_in ? base + static_cast<uint64_t>(chunks) * 64u
                                                                           : static_cast<uint64_t>(n_in);
@@ -1069,11 +1121,12 @@ __device__ __forceinline__ void transport_refill(STORM_TRANSPORT_ARGS, CensusSoA
       if (state != kAlive && state != kNone) {
         Packet<Real> p;
         p.flags = 0u;
-        tr.end(p, mesh, k, sink);
+        tr.end(p, a.mesh, a.k, sink);
+        const Args &q = args_at_use<Args>();
         if (p.ctr > longest) longest = p.ctr;
         escaped += state == kEscaped ? 1u : 0u;
-        const uint32_t oslot = wave_append(state == kPaused, n_out);
-        if (state == kPaused) store_packet(out, oslot, p);
+        const uint32_t oslot = wave_append(state == kPaused, q.n_out);
+        if (state == kPaused) store_packet(q.out, oslot, p);
         const uint64_t want = __builtin_amdgcn_ballot_w64(state == kCensus);
         if (want) {
           uint32_t first = 0u;
@@ -1081,7 +1134,7 @@ __device__ __forceinline__ void transport_refill(STORM_TRANSPORT_ARGS, CensusSoA
             first = __hip_atomic_fetch_add(cache.staged, static_cast<uint32_t>(__popcll(want)), __ATOMIC_RELAXED,
                                            __HIP_MEMORY_SCOPE_WORKGROUP);
           first = __builtin_amdgcn_readfirstlane(first);
-          if (state == kCensus) store_census(stage, static_cast<uint32_t>(base) + first + lane_rank(want), p);
+          if (state == kCensus) store_census(q.stage, static_cast<uint32_t>(base) + first + lane_rank(want), p);
         }
         state = kNone;
       }
@@ -1105,8 +1158,8 @@ __device__ __forceinline__ void transport_refill(STORM_TRANSPORT_ARGS, CensusSoA
         const uint32_t avail = pool_end - pool_next;
         const uint32_t take = nidle - given < avail ? nidle - given : avail;
         if (state != kAlive && rank >= given && rank < given + take) {
-          const Packet<Real> p = load_packet(in, static_cast<uint32_t>(base + pool_next + (rank - given)));
-          tr.begin(p, mesh, xs, k);
+          const Packet<Real> p = load_packet(args_at_use<Args>().in, static_cast<uint32_t>(base + pool_next + (rank - given)));
+          tr.begin(p, a.mesh, a.xs, a.k);
           state = kAlive;
           nseg = 0;
         }
@@ -1116,29 +1169,35 @@ __device__ __forceinline__ void transport_refill(STORM_TRANSPORT_ARGS, CensusSoA
       if (__builtin_amdgcn_ballot_w64(state == kAlive) == 0ull) break;  // the range was exhausted already
     }
     if (state == kAlive) {
-      state = tr.segment(mesh, xs, acc, k, sink);
-      if (++nseg >= max_segments && state == kAlive) state = kPaused;
+      state = tr.segment(a.mesh, a.xs, a.acc, a.k, sink);
+      if (++nseg >= a.max_segments && state == kAlive) state = kPaused;
     }
   }
-  // the staged census becomes visible to the block's last wavefront
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+  // the staged census becomes visible to the block's last wavefront (the
+  // block's wavefronts share a CU and its L1: nothing leaves the CU for it;
+  // an agent fence here would write back and invalidate the XCD's L2, once
+  // per wavefront)
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   if (sink.finish_block()) {
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     const uint32_t nst = __hip_atomic_load(cache.staged, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     uint32_t g = 0u;
-    if (nst && __lane_id() == 0u) g = atomicAdd(n_cen, nst);
+    const Args &o = args_at_use<Args>();
+    if (nst && __lane_id() == 0u) g = atomicAdd(o.n_cen, nst);
     g = __builtin_amdgcn_readfirstlane(g);
-    for (uint32_t q = __lane_id(); q < nst; q += 64u) copy_census(stage, static_cast<uint32_t>(base) + q, cen, g + q);
+    for (uint32_t q = __lane_id(); q < nst; q += 64u) copy_census(o.stage, static_cast<uint32_t>(base) + q, o.cen, g + q);
   }
+  unsigned long long *stats = args_at_use<Args>().stats;
   wave_add_u32(escaped, &stats[0]);
   wave_max_u32(longest, &stats[4]);
-  if (acc.cell) {
+  if ((F & kFeatAccel) != 0u) {
     wave_add_u32(sink.rw, &stats[1]);
     wave_add_u32(sink.ddmc, &stats[2]);
   }
 }
 
-// Waves per SIMD the refill kernel is compiled for.
+// Waves per SIMD the refill kernel is compiled for: as above (82-96 VGPRs
+// without groups, 97-118 with them).
 template <typename Real, uint32_t F, typename MeshT>
 struct RefillWaves {
   static constexpr int kMin = sizeof(Real) == 8 ? 1 : ((F & kFeatMultigroup) ? 4 : 5);
@@ -1146,11 +1205,9 @@ struct RefillWaves {
 
 template <typename Real, uint32_t F, typename MeshT = MeshView<Real>>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(RefillWaves<Real, F, MeshT>::kMin, 8))) void
-k_transport_refill(STORM_TRANSPORT_ARGS, CensusSoA<Real> stage) {
-  transport_refill<Real, F, MeshT>(n_in, in, out, n_out, cen, n_cen, mesh, xs, acc, k, max_segments, t, stats,
-                                   cache_groups, cache_fields, chunks, stage);
+k_transport_refill(TransportArgs<Real, MeshT> a) {
+  transport_refill<Real, F, MeshT>(a);
 }
-#undef STORM_TRANSPORT_ARGS
 
 // ------------------------------------------------------------------ accelerations
 // Per-cell random-walk / DDMC data (precomputeRandomWalkData, RadiationIMC.hpp:982-1063;
@@ -1964,6 +2021,45 @@ __global__ __launch_bounds__(256) void k_fold_replicas(Tallies t, uint32_t *__re
   }
   t.segs[c] = sg > 0xFFFFFFFFull ? 0xFFFFFFFFu : static_cast<uint32_t>(sg);
   if (sg >= (1ull << 28)) atomicOr(err, kErrTallyOverflow);
+}
+
+// Counts the floats among the n bit patterns from `first` on where a short
+// form of fpmath.h differs from what it stands for: 0 recip_f and 1 / x,
+// 1 sqrt_f and sqrtf, 2 log_unit and logf_d, 3 expm1_neg and expm1f_d, 4 div_f
+// and a / b for a pair made from each pattern with exponents within 2^-60 ..
+// 2^60.
+__global__ __launch_bounds__(256) void k_check_math(int32_t op, uint32_t first, uint64_t n,
+                                                    unsigned long long *__restrict__ bad) {
+  uint32_t wrong = 0u;
+  for (uint64_t i = blockIdx.x * 256ull + threadIdx.x; i < n; i += gridDim.x * 256ull) {
+    const uint32_t b = first + static_cast<uint32_t>(i);
+    const float x = fpm::u2f(b);
+    float got, want;
+    if (op == 0) {
+      got = fpm::recip_f(x);
+      want = 1.0f / x;
+    } else if (op == 1) {
+      got = fpm::sqrt_f(x);
+      want = ::sqrtf(x);
+    } else if (op == 2) {
+      got = fpm::log_unit(x);
+      want = fpm::logf_d(x);
+    } else if (op == 3) {
+      got = fpm::expm1_neg(x);
+      want = fpm::expm1f_d(x);
+    } else {
+      const Philox4 r = philox4x32_10(b, 0u, 0u, 0u, 1u, 2u);
+      auto within = [](uint32_t w, uint32_t e) {
+        return fpm::u2f((w & 0x807FFFFFu) | ((67u + e % 121u) << 23));  // 2^-60 .. 2^60
+      };
+      const float p = within(r.v[0], r.v[2]), q = within(r.v[1], r.v[3]);
+      got = fpm::div_f(p, q);
+      want = p / q;
+    }
+    wrong += fpm::f2u(got) != fpm::f2u(want) ? 1u : 0u;
+  }
+  for (int off = 32; off > 0; off >>= 1) wrong += __shfl_xor(wrong, off, 64);
+  if (wrong && __lane_id() == 0u) atomicAdd(bad, static_cast<unsigned long long>(wrong));
 }
 
 // Plain copy of n 16-byte words, one per thread: a kernel whose HBM traffic
