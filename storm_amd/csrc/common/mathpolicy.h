@@ -59,6 +59,12 @@ struct MathPolicy<double> {
   }
   STORM_HD static double sqrt_unit(double x) { return ::sqrt(x); }
   STORM_HD static void sincos2pi(double u, double &s, double &c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    // of pi times 2 u: the quadrant is exact and 2 pi u is not rounded, and
+    // there is no reduction of large arguments to carry along
+    ::sincospi(2.0 * u, &s, &c);
+    return;
+#endif
     double a = 6.283185307179586476925286766559 * u;
     s = ::sin(a);
     c = ::cos(a);

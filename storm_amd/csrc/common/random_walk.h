@@ -102,7 +102,8 @@ template <typename Real>
 STORM_HD Real sample_radius(const Tables<Real> &t, Real tau, Real xi) {
   using M = MathPolicy<Real>;
   const Real tmin = t.tau[0], tmax = t.tau[kTableSize - 1];
-  const Real tc = tau < tmin ? tmin : (tau > tmax ? tmax : tau);
+  const Real low = tau > tmax ? tmax : tau;
+  const Real tc = tau < tmin ? tmin : low;
   const Real pos = (M::log(tc) - Real(kLogTauMin)) / (Real(kLogTauMax) - Real(kLogTauMin)) * Real(kTableSize - 1);
   int ti = static_cast<int>(pos);
   if (ti > kTableSize - 2) ti = kTableSize - 2;
@@ -115,8 +116,9 @@ STORM_HD Real sample_radius(const Tables<Real> &t, Real tau, Real xi) {
   const Real xf = xp - static_cast<Real>(xj);
   const Real *r0 = t.radius + ti * kRadiusSize;
   const Real *r1 = r0 + kRadiusSize;
-  const Real a = r0[xj] + xf * (r0[xj + 1] - r0[xj]);
-  const Real b = r1[xj] + xf * (r1[xj + 1] - r1[xj]);
+  const Real a0 = r0[xj], a1 = r0[xj + 1], b0 = r1[xj], b1 = r1[xj + 1];
+  const Real a = a0 + xf * (a1 - a0);
+  const Real b = b0 + xf * (b1 - b0);
   const Real r = a + tf * (b - a);
   return r < Real(0) ? Real(0) : (r > Real(1) ? Real(1) : r);
 }

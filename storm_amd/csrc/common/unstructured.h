@@ -282,12 +282,14 @@ struct UTracker : PacketState<Real, F> {
     if constexpr ((F & kFeatAccel) != 0u) {
       if (!(Ro > Real(0))) Ro = Real(0);
       if (acc.cell && Ro >= this->r_acc) {
-        const CellAccel<Real> &ca = acc.cell[cell];
-        if ((ca.flags & 1u) && (!mg || nu < ca.e_cut) && Ro > Real(0) && ca.sig_t > Real(0) &&
-            Ro * ca.sig_t >= acc.rw_particle_tau)
-          step = kStepWalk;
-        else if ((ca.flags & 2u) && ca.total > Real(0) && Ro * ca.ddmc_sig_t >= acc.ddmc_particle_tau &&
-                 (!multigroup || nu < ca.ddmc_e_cut) && m.ddmc_rate)
+        const CellAccel<Real> ca = acc.cell[cell];
+        const bool walk = ((ca.flags & 1u) != 0u) & (!mg | (nu < ca.e_cut)) & (Ro > Real(0)) &
+                          (ca.sig_t > Real(0)) & (Ro * ca.sig_t >= acc.rw_particle_tau);
+        const bool ddmc = ((ca.flags & 2u) != 0u) & (ca.total > Real(0)) &
+                          (Ro * ca.ddmc_sig_t >= acc.ddmc_particle_tau) & (!multigroup | (nu < ca.ddmc_e_cut)) &
+                          (m.ddmc_rate != nullptr);
+        if (walk) step = kStepWalk;
+        else if (ddmc)
           step = kStepDdmc;
       }
     }
