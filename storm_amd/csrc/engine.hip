@@ -278,9 +278,7 @@ struct Engine final : EngineBase {
   DevBuf<double> wsorted;              // sorted census weights
   DevBuf<CombCell> comb_cells;
   DevBuf<int32_t> qexp;
-  // scalars read back by the host: gathered on the device, one copy into
-  // pinned memory, one synchronisation
-  DevBuf<unsigned long long> mail;
+  // scalars read back by the host: pinned, written by the device
   unsigned long long *mail_h = nullptr;
   // pinned staging of the boundary face weights (both x sides, sized at creation)
   double *wface_h = nullptr;
@@ -660,7 +658,6 @@ struct Engine final : EngineBase {
     leaving.ensure(5);  // escapes, random-walk steps, DDMC steps, segments, longest history
     dsc.ensure(3);      // material energy before the step, census energy after it, emission total
     qexp.ensure(2);     // energy quantum exponents of the step
-    mail.ensure(8);
     HIPCHECK(hipHostMalloc(reinterpret_cast<void **>(&mail_h), 8 * sizeof(unsigned long long)));
     // boundary source faces: at most both x sides of ny * nz faces
     {
@@ -994,8 +991,9 @@ struct Engine final : EngineBase {
     k_sum_partials<256><<<1, 256, 0, stream>>>(partials.p, kSumGrid, out);
   }
 
-  // Reads up to 8 device scalars (4 or 8 bytes each) with one copy into
-  // pinned memory and one synchronisation.
+  // Reads up to 8 device scalars (4 or 8 bytes each): one kernel writes them
+  // into pinned host memory (a copy would be one more launch), one
+  // synchronisation.
   const unsigned long long *read_scalars(std::initializer_list<std::pair<const void *, uint32_t>> refs) {
     ScalarRefs r{};
     uint32_t n = 0;
@@ -1004,8 +1002,7 @@ struct Engine final : EngineBase {
       r.bytes[n] = x.second;
       ++n;
     }
-    k_gather_scalars<<<1, 64, 0, stream>>>(r, n, mail.p);
-    HIPCHECK(hipMemcpyAsync(mail_h, mail.p, n * sizeof(unsigned long long), hipMemcpyDeviceToHost, stream));
+    k_gather_scalars<<<1, 64, 0, stream>>>(r, n, mail_h);
     HIPCHECK(hipStreamSynchronize(stream));
     return mail_h;
   }
@@ -1075,7 +1072,9 @@ struct Engine final : EngineBase {
       zero_flush(z);
     }
     eq_prev_ledger_ = eq_prev;
-    sum_async(e_mat.p, N, dsc.p);  // material energy before the step, read by the ledger
+    const uint32_t M = 1u << morton.total;
+    const bool small = inst.empty() && N <= kSmallCells && M <= kSmallCodes;
+    if (!small) sum_async(e_mat.p, N, dsc.p);  // material energy before the step, read by the ledger
     if (!inst.empty())
       k_inst_sum<<<static_cast<uint32_t>(inst.size()), 256, 0, stream>>>(d_inst_first.p, e_mat.p, d_inst_mat0.p);
 
@@ -1088,25 +1087,23 @@ struct Engine final : EngineBase {
           imc.with_random_walk ? imc.rw_min_cell_optical_depth : HUGE_VAL, accel_on ? accel.p : nullptr,
           (imc.with_ddmc && imc.ddmc_multigroup_pgrw) ? imc.ddmc_min_cell_optical_depth : -1.0,
           accel_on ? Dtil.p : nullptr, accelview().rw_particle_tau);
-    } else {
-      k_prestep<Real><<<blocks_for(N, 256), 256, 0, stream>>>(
-          N, T.p, md, have_host_sa ? host_sa.p : nullptr, have_host_ss ? host_ss.p : nullptr,
-          have_host_cv ? host_cv.p : nullptr, V.p, dt, xs.p, fleck.p, sig_a.p, sig_s.p, Eemit.p, err.p);
     }
-    if (accel_on && (groups < 2 || imc.with_ddmc)) {
-      k_accel_cells<Real><<<blocks_for(N, 256), 256, 0, stream>>>(
-          N, chord.p, sig_a.p, sig_s.p, fleck.p, imc.with_random_walk, imc.rw_min_cell_optical_depth, imc.with_ddmc,
-          imc.ddmc_min_cell_optical_depth, groups >= 2 ? 1 : 0, imc.ddmc_multigroup_pgrw ? 1 : 0, Dtil.p,
-          accel.p, xs.p, accelview().rw_particle_tau, accelview().ddmc_particle_tau);
-      if (unstructured) {
-        if (imc.with_ddmc)
-          k_accel_rates_u<Real><<<blocks_for(N, 256), 256, 0, stream>>>(N, u_face_start.p, u_face_nbr.p, u_face_geo.p, V.p,
-                                                                         Dtil.p, accel.p, u_ddmc_rate.p);
-      } else {
-        k_accel_rates<Real><<<blocks_for(N, 256), 256, 0, stream>>>(N, d, meshview(), Dtil.p, accel.p);
-      }
-    }
-    sum_async(Eemit.p, N, dsc.p + 2);  // emission total, read by k_quantum and k_alloc
+    PrestepArgs<Real> pre{};
+    pre.T = T.p;
+    pre.mat = md;
+    pre.host_sa = have_host_sa ? host_sa.p : nullptr;
+    pre.host_ss = have_host_ss ? host_ss.p : nullptr;
+    pre.host_cv = have_host_cv ? host_cv.p : nullptr;
+    pre.V = V.p;
+    pre.dt = dt;
+    pre.xs = xs.p;
+    pre.fleck = fleck.p;
+    pre.sig_a = sig_a.p;
+    pre.sig_s = sig_s.p;
+    pre.Eemit = Eemit.p;
+    pre.err = err.p;
+    if (groups < 2 && !small) k_prestep<Real><<<blocks_for(N, 256), 256, 0, stream>>>(N, pre);
+    if (!small) sum_async(Eemit.p, N, dsc.p + 2);  // emission total, read by k_quantum and k_alloc
 
     // boundary sources: SideTemperature / TwoSidesTemperature energy per face
     // (T^4 frozen at the first call if asked), sides x- then x+
@@ -1170,7 +1167,28 @@ struct Engine final : EngineBase {
     // energy quantum of this step (every energy below 2^62 quanta; in a batch
     // every instance's, in its own unit), photon allocation and offsets; one
     // read-back for the quantum and the count
-    if (inst.empty()) {
+    if (small) {
+      SmallStart<Real> a{};
+      a.N = N;
+      a.M = M;
+      a.pre = pre;
+      a.prestep = groups < 2 ? 1 : 0;
+      a.e_mat = e_mat.p;
+      a.dsc = dsc.p;
+      a.census_prev = census_total_prev;
+      a.source_total = source_total;
+      a.n_min = imc.new_photons_per_cell;
+      a.q = qexp.p;
+      a.nphot = nphot.p;
+      a.wemit = wemit.p;
+      a.emit_limbs = emit_limbs.p;
+      a.step = step_index;
+      a.mo = morton;
+      a.d = d;
+      a.offsets = offsets.p;
+      a.mail = mail_h;
+      k_small_start<Real><<<1, 1024, 0, stream>>>(a);
+    } else if (inst.empty()) {
       k_quantum<<<1, 64, 0, stream>>>(dsc.p + 2, census_total_prev, source_total, units::clight, dt, qexp.p);
     } else {
       const size_t K = inst.size();
@@ -1182,24 +1200,39 @@ struct Engine final : EngineBase {
       k_inst_quantum<<<1, 256, 0, stream>>>(static_cast<uint32_t>(K), d_inst_cen.p, d_inst_etot.p, d_inst_src.p,
                                              units::clight * dt, d_inst_shift.p, d_inst_shift_prev.p, qexp.p);
     }
-    k_alloc<<<blocks_for(N, 256), 256, 0, stream>>>(N, Eemit.p, dsc.p + 2, imc.new_photons_per_cell, qexp.p,
-                                                    nphot.p, wemit.p, emit_limbs.p, instview(), step_index);
-    // photon counts in the cells' Z order, so emission is laid out like the
-    // combed census
-    const uint32_t M = 1u << morton.total;
-    k_morton_counts<<<blocks_for(M + 1, 256), 256, 0, stream>>>(M, morton, d, nphot.p, nphot_z.p);
-    {
-      auto q = [&](void *tp, size_t &bytes) {
-        HIPCHECK(rocprim::exclusive_scan(tp, bytes, nphot_z.p, offsets.p, uint64_t(0), static_cast<size_t>(M) + 1,
-                                         rocprim::plus<uint64_t>(), stream));
-      };
-      ensure_temp(q);
+    if (!small) {
+      k_alloc<<<blocks_for(N, 256), 256, 0, stream>>>(N, Eemit.p, dsc.p + 2, imc.new_photons_per_cell, qexp.p,
+                                                      nphot.p, wemit.p, emit_limbs.p, instview(), step_index);
+      // photon counts in the cells' Z order, so emission is laid out like the
+      // combed census
+      k_morton_counts<<<blocks_for(M + 1, 256), 256, 0, stream>>>(M, morton, d, nphot.p, nphot_z.p);
+      {
+        auto q = [&](void *tp, size_t &bytes) {
+          HIPCHECK(rocprim::exclusive_scan(tp, bytes, nphot_z.p, offsets.p, uint64_t(0), static_cast<size_t>(M) + 1,
+                                           rocprim::plus<uint64_t>(), stream));
+        };
+        ensure_temp(q);
+      }
     }
     if (!inst.empty())
       HIPCHECK(hipMemcpyAsync(inst_shift_h, d_inst_shift.p, inst.size() * sizeof(int32_t), hipMemcpyDeviceToHost,
                               stream));
-    const unsigned long long *hs =
-        read_scalars({{offsets.p + M, 8u}, {qexp.p, 4u}, {qexp.p + 1, 4u}});
+    if (accel_on && (groups < 2 || imc.with_ddmc)) {
+      k_accel_cells<Real><<<blocks_for(N, 256), 256, 0, stream>>>(
+          N, chord.p, sig_a.p, sig_s.p, fleck.p, imc.with_random_walk, imc.rw_min_cell_optical_depth, imc.with_ddmc,
+          imc.ddmc_min_cell_optical_depth, groups >= 2 ? 1 : 0, imc.ddmc_multigroup_pgrw ? 1 : 0, Dtil.p,
+          accel.p, xs.p, accelview().rw_particle_tau, accelview().ddmc_particle_tau);
+      if (unstructured) {
+        if (imc.with_ddmc)
+          k_accel_rates_u<Real><<<blocks_for(N, 256), 256, 0, stream>>>(N, u_face_start.p, u_face_nbr.p, u_face_geo.p, V.p,
+                                                                         Dtil.p, accel.p, u_ddmc_rate.p);
+      } else {
+        k_accel_rates<Real><<<blocks_for(N, 256), 256, 0, stream>>>(N, d, meshview(), Dtil.p, accel.p);
+      }
+    }
+    const unsigned long long *hs = mail_h;
+    if (small) HIPCHECK(hipStreamSynchronize(stream));
+    else hs = read_scalars({{offsets.p + M, 8u}, {qexp.p, 4u}, {qexp.p + 1, 4u}});
     const uint64_t n_emit = hs[0];
     const int32_t eq = static_cast<int32_t>(static_cast<uint32_t>(hs[1]));
     const int32_t et = static_cast<int32_t>(static_cast<uint32_t>(hs[2]));
@@ -1330,10 +1363,8 @@ struct Engine final : EngineBase {
       HIPCHECK(hipEventRecord(ev0, stream));
       launch_transport(n_in, src, dst, mv, av, kc);
       HIPCHECK(hipEventRecord(ev1, stream));
-      HIPCHECK(hipMemcpyAsync(mail_h, counters_u32.p, 2 * sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
-      HIPCHECK(hipStreamSynchronize(stream));
-      uint32_t h[2];
-      std::memcpy(h, mail_h, sizeof h);
+      const unsigned long long *hc = read_scalars({{counters_u32.p, 4u}, {counters_u32.p + 1, 4u}});
+      const uint32_t h[2] = {static_cast<uint32_t>(hc[0]), static_cast<uint32_t>(hc[1])};
       float ms = 0.f;
       HIPCHECK(hipEventElapsedTime(&ms, ev0, ev1));
       t_transport += ms * 1e-3;
@@ -1344,7 +1375,7 @@ struct Engine final : EngineBase {
       n_cen_total = h[1];
       ping = !ping;
     }
-    k_fold_replicas<<<blocks_for(N, 256), 256, 0, stream>>>(tal, err.p);
+    if (!small) k_fold_replicas<<<blocks_for(N, 256), 256, 0, stream>>>(tal, err.p);
     counters.seconds_transport = t_transport;
     counters.seconds_transport_max_launch = t_max;
     counters.census_before_comb = n_cen_total;
@@ -1355,18 +1386,43 @@ struct Engine final : EngineBase {
     counters.end_particles = n_out;
 
     // postStep
-    k_post<Real><<<blocks_for(N, 256), 256, 0, stream>>>(
-        N, tal, eq, et, eq_prev, emit_limbs.p, requant.p, dt, V.p, md,
-        material_mode == STORM_GPU_MATERIAL_DEVICE ? 1 : 0, T.p, e_mat.p, e_sync.p, erad_avg.p, census_erad.p,
-        clamp.p, err.p, precision == STORM_GPU_FP64 ? 1 : 0, xs.p, groups >= 2 ? 0 : 1, instview());
+    PostArgs<Real> post{};
+    post.t = tal;
+    post.eq = eq;
+    post.et = et;
+    post.eq_old = eq_prev;
+    post.emit_limbs = emit_limbs.p;
+    post.requant = requant.p;
+    post.dt = dt;
+    post.V = V.p;
+    post.mat = md;
+    post.device_eos = material_mode == STORM_GPU_MATERIAL_DEVICE ? 1 : 0;
+    post.T = T.p;
+    post.e_mat = e_mat.p;
+    post.e_sync = e_sync.p;
+    post.erad_avg = erad_avg.p;
+    post.census_erad = census_erad.p;
+    post.clamp = clamp.p;
+    post.err = err.p;
+    post.fp64 = precision == STORM_GPU_FP64 ? 1 : 0;
+    post.xs = xs.p;
+    post.gray = groups >= 2 ? 0 : 1;
+    post.inst = instview();
     // census energy for the next step's quantum, total segments, error flags
     // and counters: one synchronisation
-    sum_async(census_erad.p, N, dsc.p + 1);
-    if (!inst.empty())
-      k_inst_sum<<<static_cast<uint32_t>(inst.size()), 256, 0, stream>>>(d_inst_first.p, census_erad.p, d_inst_cen.p);
-    k_total_u32<<<std::min<uint32_t>(blocks_for(N, 256), 1024u), 256, 0, stream>>>(N, tal.segs, leaving.p + 3);
-    const unsigned long long *hp = read_scalars({{dsc.p + 1, 8u}, {err.p, 4u}, {leaving.p, 8u}, {leaving.p + 1, 8u},
-                                                 {leaving.p + 2, 8u}, {leaving.p + 3, 8u}, {leaving.p + 4, 8u}});
+    const unsigned long long *hp = mail_h;
+    if (small) {
+      k_small_end<Real><<<1, 1024, 0, stream>>>(N, post, dsc.p, leaving.p, mail_h);
+      HIPCHECK(hipStreamSynchronize(stream));
+    } else {
+      k_post<Real><<<blocks_for(N, 256), 256, 0, stream>>>(N, post);
+      sum_async(census_erad.p, N, dsc.p + 1);
+      if (!inst.empty())
+        k_inst_sum<<<static_cast<uint32_t>(inst.size()), 256, 0, stream>>>(d_inst_first.p, census_erad.p, d_inst_cen.p);
+      k_total_u32<<<std::min<uint32_t>(blocks_for(N, 256), 1024u), 256, 0, stream>>>(N, tal.segs, leaving.p + 3);
+      hp = read_scalars({{dsc.p + 1, 8u}, {err.p, 4u}, {leaving.p, 8u}, {leaving.p + 1, 8u}, {leaving.p + 2, 8u},
+                         {leaving.p + 3, 8u}, {leaving.p + 4, 8u}});
+    }
     const double hcensus = as_double(hp[0]);
     const uint32_t herr = static_cast<uint32_t>(hp[1]);
     unsigned long long hstats[5];
@@ -1416,7 +1472,6 @@ struct Engine final : EngineBase {
     f(counters_u32);
     f(err);
     f(qexp);
-    f(mail);
     f(leaving);
   }
   template <typename F>
@@ -1447,7 +1502,7 @@ struct Engine final : EngineBase {
     f(offs64);
     f(temp);
   }
-  static constexpr size_t kTransientBufs = 6 + 2 * 5 + 4 + 4 + 10;
+  static constexpr size_t kTransientBufs = 5 + 2 * 5 + 4 + 4 + 10;
 
   void step_noalloc(double dt) override {
     if (keep_inputs)

@@ -283,29 +283,37 @@ __global__ __launch_bounds__(256) void k_morton_counts(uint32_t M, Morton mo, Me
 
 
 // ------------------------------------------------------------------ preStep
+// Where a step's material comes from and what preStep makes of it, per cell.
 template <typename Real>
-__global__ __launch_bounds__(256) void k_prestep(uint32_t N, const double *__restrict__ T, MatDev mat,
-                                                 const double *__restrict__ host_sa,
-                                                 const double *__restrict__ host_ss,
-                                                 const double *__restrict__ host_cv,
-                                                 const double *__restrict__ V, double dt,
-                                                 CellXS<Real> *__restrict__ xs, double *__restrict__ fleck,
-                                                 double *__restrict__ sig_a_out, double *__restrict__ sig_s_out,
-                                                 double *__restrict__ Eemit, uint32_t *__restrict__ err) {
-  uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= N) return;
-  const double Tc = T[c];
-  const double sa = host_sa ? host_sa[c] : mat.sigma_a(c, Tc);
-  const double ss = host_ss ? host_ss[c] : mat.sigma_s(c, Tc);
-  const double cv = host_cv ? host_cv[c] : mat.dT2cv(mat.density(c), Tc);
+struct PrestepArgs {
+  const double *T;
+  MatDev mat;
+  const double *host_sa, *host_ss, *host_cv;
+  const double *V;
+  double dt;
+  CellXS<Real> *xs;
+  double *fleck, *sig_a, *sig_s, *Eemit;
+  uint32_t *err;
+};
+template <typename Real>
+__device__ __forceinline__ void prestep_cell(uint32_t c, const PrestepArgs<Real> &a) {
+  const double Tc = a.T[c];
+  const double sa = a.host_sa ? a.host_sa[c] : a.mat.sigma_a(c, Tc);
+  const double ss = a.host_ss ? a.host_ss[c] : a.mat.sigma_s(c, Tc);
+  const double cv = a.host_cv ? a.host_cv[c] : a.mat.dT2cv(a.mat.density(c), Tc);
   const double T3 = Tc * Tc * Tc;
-  const double f = 1.0 / (1.0 + (4.0 * units::arad * T3 * sa * units::clight * dt) / cv);
-  if (!(f >= 0.0 && f <= 1.0)) atomicOr(err, kErrFleck);
-  fleck[c] = f;
-  sig_a_out[c] = sa;
-  sig_s_out[c] = ss;
-  Eemit[c] = f * V[c] * units::arad * (T3 * Tc) * sa * dt * units::clight;
-  xs[c] = make_xs<Real>(static_cast<Real>(f * sa), static_cast<Real>(ss + (1.0 - f) * sa));
+  const double f = 1.0 / (1.0 + (4.0 * units::arad * T3 * sa * units::clight * a.dt) / cv);
+  if (!(f >= 0.0 && f <= 1.0)) atomicOr(a.err, kErrFleck);
+  a.fleck[c] = f;
+  a.sig_a[c] = sa;
+  a.sig_s[c] = ss;
+  a.Eemit[c] = f * a.V[c] * units::arad * (T3 * Tc) * sa * a.dt * units::clight;
+  a.xs[c] = make_xs<Real>(static_cast<Real>(f * sa), static_cast<Real>(ss + (1.0 - f) * sa));
+}
+template <typename Real>
+__global__ __launch_bounds__(256) void k_prestep(uint32_t N, PrestepArgs<Real> a) {
+  const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
+  if (c < N) prestep_cell<Real>(c, a);
 }
 
 // Multigroup preStep per cell (storm_group_desc): the Planck opacity
@@ -440,12 +448,16 @@ __global__ __launch_bounds__(256) void k_prestep_mg(
 // census energy of the last step, this step's emission total and the boundary
 // source total) is below 2^62 quanta; q[0] for energies, q[1] for path
 // integrals (energy x c dt).  The host reads them back.
+__device__ __forceinline__ void step_quantum(double Etot, double census_prev, double source_total, double c, double dt,
+                                             int32_t *__restrict__ q) {
+  const double Ebound = census_prev + Etot + source_total;
+  q[0] = Ebound > 0.0 ? fx::ceil_log2(Ebound) - fx::kHeadroomBits : -1000;
+  q[1] = Ebound > 0.0 ? fx::ceil_log2(Ebound * c * dt) - fx::kHeadroomBits : -1000;
+}
 __global__ void k_quantum(const double *__restrict__ Etot, double census_prev, double source_total, double c,
                           double dt, int32_t *__restrict__ q) {
   if (threadIdx.x != 0u || blockIdx.x != 0u) return;
-  const double Ebound = census_prev + *Etot + source_total;
-  q[0] = Ebound > 0.0 ? fx::ceil_log2(Ebound) - fx::kHeadroomBits : -1000;
-  q[1] = Ebound > 0.0 ? fx::ceil_log2(Ebound * c * dt) - fx::kHeadroomBits : -1000;
+  step_quantum(*Etot, census_prev, source_total, c, dt, q);
 }
 
 // Batches of independent instances (inst.cell non-null).  Each instance counts energy in its own unit, 2^-shift erg (shift >= 0, set
@@ -508,24 +520,9 @@ __global__ __launch_bounds__(256) void k_inst_quantum(uint32_t K, const double *
 // photons per cell and packet weight, rounded to the step quantum without bias.
 // Batches: each instance allocates over its own cells with its own
 // newPhotonsPerCell and emission total, weights in its unit.
-__global__ __launch_bounds__(256) void k_alloc(uint32_t N, const double *__restrict__ Eemit,
-                                               const double *__restrict__ Etot_p, uint64_t n_min_all,
-                                               const int32_t *__restrict__ q, uint32_t *__restrict__ nphot,
-                                               double *__restrict__ wemit,
-                                               unsigned long long *__restrict__ emit_limbs, InstanceView inst,
-                                               uint32_t step) {
-  uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= N) return;
-  double Etot = *Etot_p;
-  uint64_t Ncells = N, n_min = n_min_all;
-  if (inst.cell) {
-    const uint32_t k = inst.cell[c];
-    Etot = inst.etot[k];
-    Ncells = inst.ncells[k];
-    n_min = inst.nphot[k];
-  }
-  const int32_t eq = q[0];
-  const double E = Eemit[c];
+__device__ __forceinline__ void alloc_cell(uint32_t c, double E, double Etot, uint64_t Ncells, uint64_t n_min,
+                                           int32_t eq, int32_t shift, uint32_t step, uint32_t *__restrict__ nphot,
+                                           double *__restrict__ wemit, unsigned long long *__restrict__ emit_limbs) {
   const uint64_t total = Ncells * n_min * 10ull;
   uint64_t share = Etot > 0.0 ? static_cast<uint64_t>(E / Etot * static_cast<double>(total)) : n_min;
   uint64_t n = 0;
@@ -536,7 +533,7 @@ __global__ __launch_bounds__(256) void k_alloc(uint32_t N, const double *__restr
   double w = 0.0;
   if (n) {
     const double per = E / static_cast<double>(n);
-    w = fx::emission_round(inst.cell ? ldexp(per, inst.shift[inst.cell[c]]) : per, eq, c, step);
+    w = fx::emission_round(shift ? ldexp(per, shift) : per, eq, c, step);
   }
   if (w == 0.0) n = 0;  // below one quantum: nothing to emit
   nphot[c] = static_cast<uint32_t>(n);
@@ -544,6 +541,134 @@ __global__ __launch_bounds__(256) void k_alloc(uint32_t N, const double *__restr
   fx::Limbs L = n ? fx::limbs_of(w, eq) : fx::Limbs{0, 0};
   emit_limbs[2 * c] = L.lo * n;
   emit_limbs[2 * c + 1] = L.hi * n;
+}
+__global__ __launch_bounds__(256) void k_alloc(uint32_t N, const double *__restrict__ Eemit,
+                                               const double *__restrict__ Etot_p, uint64_t n_min_all,
+                                               const int32_t *__restrict__ q, uint32_t *__restrict__ nphot,
+                                               double *__restrict__ wemit,
+                                               unsigned long long *__restrict__ emit_limbs, InstanceView inst,
+                                               uint32_t step) {
+  uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
+  if (c >= N) return;
+  double Etot = *Etot_p;
+  uint64_t Ncells = N, n_min = n_min_all;
+  int32_t shift = 0;
+  if (inst.cell) {
+    const uint32_t k = inst.cell[c];
+    Etot = inst.etot[k];
+    Ncells = inst.ncells[k];
+    n_min = inst.nphot[k];
+    shift = inst.shift[k];
+  }
+  alloc_cell(c, Eemit[c], Etot, Ncells, n_min, q[0], shift, step, nphot, wemit, emit_limbs);
+}
+
+// Sum of d[0 .. n) for n <= 4096 in the order k_sum_partials adds (512 blocks
+// of 256, then one of 256: partial sums of 256 in a row by a tree, and these by
+// a tree), by one block of 1024 threads; the result in every thread.  `sh`:
+// 1024 doubles.
+__device__ __forceinline__ double block_sum_in_order(const double *__restrict__ d, uint32_t n, double *sh) {
+  __shared__ double part[16];
+  const uint32_t t = threadIdx.x & 255u, g = threadIdx.x >> 8;
+  if (threadIdx.x < 16u) part[threadIdx.x] = 0.0;
+  for (uint32_t b0 = 0; b0 * 256u < n; b0 += 4u) {
+    const uint32_t i = (b0 + g) * 256u + t;
+    sh[threadIdx.x] = i < n ? 0.0 + d[i] : 0.0;
+    __syncthreads();
+    for (uint32_t s = 128u; s > 0u; s >>= 1) {
+      if (t < s) sh[threadIdx.x] += sh[threadIdx.x + s];
+      __syncthreads();
+    }
+    if (t == 0u && b0 + g < 16u) part[b0 + g] = sh[threadIdx.x];
+    __syncthreads();
+  }
+  double p[16];
+  for (uint32_t k = 0; k < 16u; ++k) p[k] = part[k];
+  for (uint32_t s = 8u; s > 0u; s >>= 1)
+    for (uint32_t k = 0; k < s; ++k) p[k] += p[k + s];
+  __syncthreads();
+  return p[0];
+}
+
+// The start of a step of a small problem (at most 4096 cells and 8192 Z-order
+// codes, not a batch) in one launch instead of ten: material energy, preStep
+// (gray; `prestep` null: done already), emission total, quantum, photon
+// allocation, the counts in Z order and their offsets, and the three numbers
+// the host waits for, written straight to its pinned mailbox.  Each of those
+// launches runs a few us of work behind about 5 us of launching and waiting
+// for the one before, which is most of a small problem's step (100 cells, 1e5
+// packets: 47 launches, 0.39 ms, of which 0.11 are the transport).  One block:
+// the parts depend on each other through sums over all cells.
+constexpr uint32_t kSmallCells = 4096, kSmallCodes = 8192;
+template <typename Real>
+struct SmallStart {
+  uint32_t N, M;
+  PrestepArgs<Real> pre;
+  int32_t prestep;
+  const double *e_mat;
+  double *dsc;  // [0] material energy, [2] emission total
+  double census_prev, source_total;
+  uint64_t n_min;
+  int32_t *q;
+  uint32_t *nphot;
+  double *wemit;
+  unsigned long long *emit_limbs;
+  uint32_t step;
+  Morton mo;
+  MeshDims d;
+  uint64_t *offsets;
+  unsigned long long *mail;
+};
+template <typename Real>
+__global__ __launch_bounds__(1024) void k_small_start(SmallStart<Real> a) {
+  __shared__ double sh[1024];
+  __shared__ uint64_t wave_sum[16];
+  __shared__ int32_t eq_s;
+  const uint32_t tid = threadIdx.x;
+  if (a.prestep)
+    for (uint32_t c = tid; c < a.N; c += 1024u) prestep_cell<Real>(c, a.pre);
+  const double mat = block_sum_in_order(a.e_mat, a.N, sh);
+  __syncthreads();  // the emission energies of every thread
+  const double Etot = block_sum_in_order(a.pre.Eemit, a.N, sh);
+  if (tid == 0u) {
+    a.dsc[0] = mat;
+    a.dsc[2] = Etot;
+    step_quantum(Etot, a.census_prev, a.source_total, units::clight, a.pre.dt, a.q);
+    eq_s = a.q[0];
+    a.mail[1] = static_cast<uint32_t>(a.q[0]);
+    a.mail[2] = static_cast<uint32_t>(a.q[1]);
+  }
+  __syncthreads();
+  for (uint32_t c = tid; c < a.N; c += 1024u)
+    alloc_cell(c, a.pre.Eemit[c], Etot, a.N, a.n_min, eq_s, 0, a.step, a.nphot, a.wemit, a.emit_limbs);
+  __syncthreads();
+  // exclusive scan of the counts over the codes: each thread a run of them
+  const uint32_t per = (a.M + 1023u) / 1024u, first = tid * per;
+  auto count = [&](uint32_t code) -> uint32_t {
+    if (code >= a.M) return 0u;
+    uint32_t i, j, k;
+    morton_ijk(code, a.mo, i, j, k);
+    return (i < a.d.nx && j < a.d.ny && k < a.d.nz) ? a.nphot[(i * a.d.ny + j) * a.d.nz + k] : 0u;
+  };
+  uint64_t own = 0;
+  for (uint32_t q = 0; q < per; ++q) own += count(first + q);
+  uint64_t incl = own;
+  for (uint32_t off = 1; off < 64u; off <<= 1) {
+    const uint64_t o = __shfl_up(static_cast<unsigned long long>(incl), off, 64);
+    if (__lane_id() >= off) incl += o;
+  }
+  if (__lane_id() == 63u) wave_sum[tid >> 6] = incl;
+  __syncthreads();
+  uint64_t at = incl - own;
+  for (uint32_t w = 0; w < (tid >> 6); ++w) at += wave_sum[w];
+  for (uint32_t q = 0; q < per; ++q) {
+    if (first + q < a.M) a.offsets[first + q] = at;
+    at += count(first + q);
+  }
+  if (tid == 1023u) {
+    a.offsets[a.M] = at;
+    a.mail[0] = at;
+  }
 }
 
 // ------------------------------------------------------------------ sourcing
@@ -1864,19 +1989,27 @@ __global__ __launch_bounds__(256) void k_comb_write(uint32_t n, const uint32_t *
 
 // ------------------------------------------------------------------ postStep
 template <typename Real>
-__global__ __launch_bounds__(256) void k_post(uint32_t N, Tallies t, int32_t eq, int32_t et, int32_t eq_old,
-                                              const unsigned long long *__restrict__ emit_limbs,
-                                              const unsigned long long *__restrict__ requant, double dt,
-                                              const double *__restrict__ V, MatDev mat, int32_t device_eos,
-                                              double *__restrict__ T, double *__restrict__ e_mat,
-                                              double *__restrict__ e_sync, double *__restrict__ erad_avg,
-                                              double *__restrict__ census_erad, double *__restrict__ clamp,
-                                              uint32_t *__restrict__ err, int32_t fp64,
-                                              const CellXS<Real> *__restrict__ xs, int32_t gray,
-                                              InstanceView inst) {
-  uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= N) return;
-  if (*err & kErrTallyOverflow) return;  // the step's tallies are not trusted: commit nothing
+struct PostArgs {
+  Tallies t;
+  int32_t eq, et, eq_old;
+  const unsigned long long *emit_limbs, *requant;
+  double dt;
+  const double *V;
+  MatDev mat;
+  int32_t device_eos;
+  double *T, *e_mat, *e_sync, *erad_avg, *census_erad, *clamp;
+  uint32_t *err;
+  int32_t fp64;
+  const CellXS<Real> *xs;
+  int32_t gray;
+  InstanceView inst;
+};
+template <typename Real>
+__device__ __forceinline__ void post_cell(uint32_t c, const PostArgs<Real> &a) {
+  const Tallies &t = a.t;
+  int32_t eq = a.eq, et = a.et, eq_old = a.eq_old;
+  const MatDev &mat = a.mat;
+  const InstanceView &inst = a.inst;
   int32_t sh = 0;  // batches: the cell's instance unit is 2^-sh erg (2^-sh_prev for the census' requant)
   if (inst.cell) {
     const uint32_t k = inst.cell[c];
@@ -1885,9 +2018,9 @@ __global__ __launch_bounds__(256) void k_post(uint32_t N, Tallies t, int32_t eq,
     eq -= sh;
     et -= sh;
   }
-  const double emit = fx::to_double(emit_limbs[2 * c], emit_limbs[2 * c + 1], eq);
+  const double emit = fx::to_double(a.emit_limbs[2 * c], a.emit_limbs[2 * c + 1], eq);
   double dep, pint;
-  if (fp64) {
+  if (a.fp64) {
     dep = ldexp(t.dep_fp[c], -sh);
     pint = ldexp(t.pint_fp[c], -sh);
   } else {
@@ -1895,36 +2028,43 @@ __global__ __launch_bounds__(256) void k_post(uint32_t N, Tallies t, int32_t eq,
     // Each segment absorbs w (1 - e^{-x}) and adds w (1 - e^{-x}) / sig_abs to
     // the path integral, so where sig_abs > 0 the integral is the absorbed
     // energy over sig_abs (the transport skips that tally there).
-    const double sabs = static_cast<double>(xs[c].sig_abs);
-    pint = (gray && sabs > 0.0) ? dep / sabs : fx::to_double(t.pint[2 * c], t.pint[2 * c + 1], et);
+    const double sabs = static_cast<double>(a.xs[c].sig_abs);
+    pint = (a.gray && sabs > 0.0) ? dep / sabs : fx::to_double(t.pint[2 * c], t.pint[2 * c + 1], et);
     dep += fx::to_double(t.rdep[2 * c], t.rdep[2 * c + 1], eq);
   }
   dep += fx::to_double(t.rem[2 * c], t.rem[2 * c + 1], eq);
-  dep += fx::to_double(requant[2 * c], requant[2 * c + 1], eq_old);
-  const double Vc = V[c];
-  erad_avg[c] = pint / (units::clight * dt * Vc);  // RadiationIMC.hpp:1895 (time integral = path / c)
-  census_erad[c] = fx::to_double(t.cout[2 * c], t.cout[2 * c + 1], eq);
-  double E = (e_mat[c] - emit) + dep;
+  dep += fx::to_double(a.requant[2 * c], a.requant[2 * c + 1], eq_old);
+  const double Vc = a.V[c];
+  a.erad_avg[c] = pint / (units::clight * a.dt * Vc);  // RadiationIMC.hpp:1895 (time integral = path / c)
+  a.census_erad[c] = fx::to_double(t.cout[2 * c], t.cout[2 * c + 1], eq);
+  double E = (a.e_mat[c] - emit) + dep;
   double cl = 0.0;
   if (E < 0.0) {  // throwIfNegativeInternalEnergy (RadiationIMC.hpp:771-817)
-    const double Tc = T[c];
+    const double Tc = a.T[c];
     double thermal = units::arad * (Tc * Tc * Tc * Tc) * Vc;
     if (thermal < 1e-30) thermal = 1e-30;
     if (fabs(E) / thermal < 0.1) {
-      double ne = fmax(0.0, e_sync[c]);
+      double ne = fmax(0.0, a.e_sync[c]);
       cl = ne - E;
       E = ne;
     } else {
-      atomicOr(err, kErrNegativeEnergy);
+      atomicOr(a.err, kErrNegativeEnergy);
     }
   }
-  clamp[c] = cl;
-  e_mat[c] = E;
-  e_sync[c] = E;
-  if (device_eos) {
+  a.clamp[c] = cl;
+  a.e_mat[c] = E;
+  a.e_sync[c] = E;
+  if (a.device_eos) {
     const double rho = mat.density(c);
-    T[c] = mat.de2T(rho, E / (rho * Vc));  // synchronizeMaterialCell (:830-866)
+    a.T[c] = mat.de2T(rho, E / (rho * Vc));  // synchronizeMaterialCell (:830-866)
   }
+}
+template <typename Real>
+__global__ __launch_bounds__(256) void k_post(uint32_t N, PostArgs<Real> a) {
+  const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
+  if (c >= N) return;
+  if (*a.err & kErrTallyOverflow) return;  // the step's tallies are not trusted: commit nothing
+  post_cell<Real>(c, a);
 }
 
 // out[0] += sum of v[0..N) (integer, order independent)
@@ -2001,9 +2141,8 @@ __device__ __forceinline__ void fold_record(const Tallies &t, uint32_t c, T v[3]
     v[2] += e[t.rec_words == 4u ? 2 : 1];
   }
 }
-__global__ __launch_bounds__(256) void k_fold_replicas(Tallies t, uint32_t *__restrict__ err) {
-  const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= t.ncell) return;
+// Returns the cell's segments; `overflow`: more of them than its tallies hold.
+__device__ __forceinline__ uint32_t fold_cell(const Tallies &t, uint32_t c, bool &overflow) {
   uint64_t sg;
   if (t.dep_fp) {
     double v[3];
@@ -2020,7 +2159,56 @@ __global__ __launch_bounds__(256) void k_fold_replicas(Tallies t, uint32_t *__re
     sg = v[2];
   }
   t.segs[c] = sg > 0xFFFFFFFFull ? 0xFFFFFFFFu : static_cast<uint32_t>(sg);
-  if (sg >= (1ull << 28)) atomicOr(err, kErrTallyOverflow);
+  overflow = sg >= (1ull << 28);
+  return t.segs[c];
+}
+__global__ __launch_bounds__(256) void k_fold_replicas(Tallies t, uint32_t *__restrict__ err) {
+  const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
+  bool overflow = false;
+  if (c < t.ncell) fold_cell(t, c, overflow);
+  if (overflow) atomicOr(err, kErrTallyOverflow);
+}
+
+// The end of a step of a small problem (at most kSmallCells cells, not a
+// batch) in one launch instead of six (see k_small_start): the replicas'
+// sums, postStep, the census energy, the segments, and the numbers the host
+// reads, into its pinned mailbox: census energy, error flags, and stats[0..4]
+// with the segments in [3].
+template <typename Real>
+__global__ __launch_bounds__(1024) void k_small_end(uint32_t N, PostArgs<Real> a, double *__restrict__ dsc,
+                                                    unsigned long long *__restrict__ stats,
+                                                    unsigned long long *__restrict__ mail) {
+  __shared__ double sh[1024];
+  __shared__ unsigned long long segs_s;
+  const uint32_t tid = threadIdx.x;
+  if (tid == 0u) segs_s = 0ull;
+  __syncthreads();
+  unsigned long long sg = 0;
+  bool overflow = (*a.err & kErrTallyOverflow) != 0u;
+  for (uint32_t c = tid; c < N; c += 1024u) {
+    bool o;
+    sg += fold_cell(a.t, c, o);
+    overflow |= o;
+  }
+  for (int off = 32; off > 0; off >>= 1) sg += __shfl_xor(sg, off, 64);
+  if (__lane_id() == 0u && sg) atomicAdd(&segs_s, sg);
+  overflow = __syncthreads_or(overflow);
+  if (!overflow)  // else the step's tallies are not trusted: commit nothing
+    for (uint32_t c = tid; c < N; c += 1024u) post_cell<Real>(c, a);
+  else if (tid == 0u)
+    atomicOr(a.err, kErrTallyOverflow);
+  __threadfence();  // every thread's error flags are set before thread 0 reads them
+  __syncthreads();
+  const double census = block_sum_in_order(a.census_erad, N, sh);
+  if (tid == 0u) {
+    dsc[1] = census;
+    stats[3] = segs_s;
+    unsigned long long bits;
+    __builtin_memcpy(&bits, &census, sizeof bits);
+    mail[0] = bits;
+    mail[1] = __hip_atomic_load(a.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int k = 0; k < 5; ++k) mail[2 + k] = k == 3 ? segs_s : stats[k];
+  }
 }
 
 // Counts the floats among the n bit patterns from `first` on where a short
