@@ -301,7 +301,7 @@ def c4_line(W, K, log, fp64=True):
                value=m["segments"] / m["wall"], unit="segments/s", steps=K, warmup=W,
                ms_per_step=m["wall"] / K * 1e3, packets_per_step=m["packets"] / K,
                segments_per_step=m["segments"] / K, transport_segments_per_s=m["segments"] / m["transport"],
-               faces=int(mesh.nfaces), kernel="k_transport<float, 2u, UMeshView<float>> (multigroup)")
+               faces=int(mesh.nfaces), kernel="k_transport_refill<float, 2u, UMeshView<float>> (multigroup)")
     if fp64:
         f = _run_steps(spec, capi.FP64, W + K, W, log, "c4 fp64")
         out["fp64_gpu"] = dict(value=f["segments"] / f["wall"], ms_per_step=f["wall"] / K * 1e3,

@@ -226,15 +226,18 @@ int storm_gpu_queue_source_packets(storm_gpu_engine *eng, const storm_packet_rec
  * (-1: keep the engine's).  PASS runs each lane's packet to its end (or the
  * segment budget) before the wavefront takes the next 64 of the block's
  * range; REFILL advances the wavefront's packets one segment at a time and
- * hands lanes whose packet ended the next packets of the block's range, four
+ * hands lanes whose packet ended the next packets of the block's range, eight
  * or more lanes at a time.  A block's range is block size x chunks per
  * wavefront (storm_gpu_set_chunks_per_wave; each schedule keeps its own,
  * 2 for PASS and 8 for REFILL by default, 16 for REFILL in the FP64 engine;
  * in the mixed engine on polyhedral meshes 4 for REFILL, and 1 for PASS on
  * multigroup problems; 16 for REFILL, in 512-thread blocks, on Cartesian
- * problems with DDMC; blocks are otherwise 256 threads; a launch halves
- * it while it would have fewer blocks than the device holds at once).  The engine starts in REFILL, except the mixed engine
- * on multigroup polyhedral problems (PASS), and watches: after 16 steps one
+ * problems with DDMC; blocks are otherwise 256 threads; a launch takes 8 for
+ * 16 when it would be less than two and a half rounds of the blocks that the
+ * device holds at once, and halves it while it would be less than one).  The
+ * engine starts in REFILL (storm_gpu_step_noalloc runs multigroup polyhedral
+ * problems of the mixed engine in PASS, which needs less scratch, unless the
+ * launch was set or is being tuned) and watches: after 16 steps one
  * step runs in the other schedule, and the engine switches when that one
  * moved more transport segments per second than the mean of the steps
  * either side of it, by more than 3%; the next probe follows 16 steps later,

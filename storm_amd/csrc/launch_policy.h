@@ -78,10 +78,9 @@ struct LaunchPolicy {
 
   // The schedule watch.  The workload of a problem changes as it runs (a
   // cold start that the random walk dominates, a heated region that then
-  // spreads), and so may the faster schedule (with a refill kernel compiled
-  // for 6 waves per SIMD, refill was 24% faster on the 64^3 cube over steps
-  // 3-12 and pass 12% faster over steps 13-50; at 5 waves refill leads
-  // throughout).  Every watch_every steps one step runs in the other
+  // spreads), and so may the faster schedule (refill leads on the large
+  // problems measured, 6.1 against 11.5 ms a step on the 64^3 cube; on the
+  // 100-cell slab of 1e5 packets pass is about 10% faster).  Every watch_every steps one step runs in the other
   // schedule; its rate is compared with the mean of the steps either side of
   // it (which cancels a steady trend) and the engine switches when the other
   // is more than 3% faster.  A probe that loses by more than 10% doubles the
