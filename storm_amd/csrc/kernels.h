@@ -590,7 +590,7 @@ __device__ __forceinline__ double block_sum_in_order(const double *__restrict__ 
   return p[0];
 }
 
-// The start of a step of a small problem (at most 4096 cells and 8192 Z-order
+// The start of a step of a small problem (at most 2048 cells and 4096 Z-order
 // codes, not a batch) in one launch instead of ten: material energy, preStep
 // (gray; `prestep` null: done already), emission total, quantum, photon
 // allocation, the counts in Z order and their offsets, and the three numbers
@@ -598,8 +598,13 @@ __device__ __forceinline__ double block_sum_in_order(const double *__restrict__ 
 // launches runs a few us of work behind about 5 us of launching and waiting
 // for the one before, which is most of a small problem's step (100 cells, 1e5
 // packets: 47 launches, 0.39 ms, of which 0.11 are the transport).  One block:
-// the parts depend on each other through sums over all cells.
-constexpr uint32_t kSmallCells = 4096, kSmallCodes = 8192;
+// the parts depend on each other through sums over all cells.  The limits are
+// where one block's passes over the cells cost what the launches did (us of a
+// step outside the transport, general path / one block: 100 cells 196/152,
+// 1000 217/187, 2000 234/225, 4096 294/317; 12^3 cells, 4096 codes, 241/218,
+// 16^3 247/272).
+constexpr uint32_t kSmallCells = 2048, kSmallCodes = 4096;
+static_assert(kSmallCells <= 4096, "block_sum_in_order");
 template <typename Real>
 struct SmallStart {
   uint32_t N, M;

@@ -1,4 +1,4 @@
-"""Steps whose start and end run as one block each (up to 4096 cells and 8192
+"""Steps whose start and end run as one block each (up to 2048 cells and 4096
 Z-order codes) and steps on either side of that line.
 
 Both routes have to give the same numbers: the photon allocation worked out
@@ -17,9 +17,10 @@ from storm_amd.engine import GpuEngine
 pytestmark = pytest.mark.gpu
 
 N_MIN = 7
-# cells: 1, a wavefront less one, a block, one more, the limit, one more (241 * 17, 8192 codes), the limit as a
-# cube; then 8192 codes for 1755 cells and 16384 for 2805
-SHAPES = [(1, 1, 1), (63, 1, 1), (1024, 1, 1), (1025, 1, 1), (4096, 1, 1), (241, 17, 1), (16, 16, 16), (3, 5, 7),
+# cells: 1, a wavefront less one, a block, one more, the limit, one more; 729 cells with the most codes, 1377 with
+# more; a cube, lines and slabs beyond
+SHAPES = [(1, 1, 1), (63, 1, 1), (1024, 1, 1), (1025, 1, 1), (2048, 1, 1), (2049, 1, 1), (9, 9, 9), (17, 9, 9),
+          (4096, 1, 1), (241, 17, 1), (16, 16, 16), (3, 5, 7),
           (65, 9, 3), (33, 17, 5)]
 
 
