@@ -103,3 +103,17 @@ def test_noalloc_step_rejects_the_debug_input_copy():
         e.keep_transport_inputs(True)
         with pytest.raises(StormError, match="error 1"):
             e.step_noalloc()
+
+
+def test_noalloc_multigroup_voronoi_runs_passes():
+    """The refill schedule, this problem's default, stages its census in the
+    scratch; without an allocation it runs passes, with the same results."""
+    spec = P.c4_voronoi(seed=15, n=500, groups=8, steps=2, packets_scale=0.005)
+    with GpuEngine(spec, capi.MIXED) as ref, GpuEngine(spec, capi.MIXED) as na:
+        for step in range(spec.steps):
+            ref.step()
+            na.step_noalloc()
+            assert ref.counters()["transport_schedule"] == capi.SCHEDULE_REFILL
+            assert na.counters()["transport_schedule"] == capi.SCHEDULE_PASS
+            assert na.launch()["schedule"] == capi.SCHEDULE_REFILL
+            _assert_same(_state(ref), _state(na), f"step {step + 1}")
