@@ -1398,7 +1398,7 @@ struct Engine final : EngineBase {
       ping = !ping;
     }
     hold.end();
-    if (!small) k_fold_replicas<<<blocks_for(N, 256), 256, 0, stream>>>(tal, err.p);
+    if (!small) k_fold_replicas<Real><<<blocks_for(N, 256), 256, 0, stream>>>(tal, xs.p, err.p);
     counters.seconds_transport = t_transport;
     counters.seconds_transport_max_launch = t_max;
     counters.census_before_comb = n_cen_total;

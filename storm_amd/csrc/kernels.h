@@ -141,8 +141,10 @@ struct Tallies {
   uint32_t *begin;           // [N]  packets per cell at transport start
   // The per-visit tallies while the transport runs, one record of `rec_words`
   // 64-bit words per cell and XCD, [replica][cell]: the deposit, the path
-  // integral (not with 2 words) and the segments, as integers in the mixed
-  // engine and doubles in the FP64 engine.  A wavefront adds into the replica
+  // integral and the segments, as integers in the mixed engine and doubles in
+  // the FP64 engine.  With 2 words (mixed gray engine) the first is the path
+  // integral in cells without absorption, where the deposit is 0, and the
+  // deposit elsewhere, where postStep derives the path integral from it.  A wavefront adds into the replica
   // of the XCD it runs on, so that the atomics of different XCDs never share
   // a cache line; k_fold_replicas sums them into dep, pint and segs above.
   // One record per cell because an atomic costs what the 64-byte line it
@@ -870,8 +872,8 @@ __global__ __launch_bounds__(256) void k_boundary(uint32_t n_bc, uint32_t npc, c
 // (doubles in v[0], v[1]) change only their order.
 // The table lives in dynamic LDS: `groups` groups of four slots of `nf`
 // 64-bit sums, a tag and a segment count each.  nf = 1 in the mixed gray
-// engine (the deposit, in quanta; the path integral, tallied only in cells
-// without absorption, goes to device memory), 2 in the mixed multigroup
+// engine (the deposit or, in cells without absorption, the path integral, in
+// quanta: Tallies::rec), 2 in the mixed multigroup
 // engine (deposit and path integral), 2 in the FP64 engine (deposit and
 // path integral as doubles).  Four cells in a row hash to one group, so that
 // the records of a group lie in one or two 64-byte lines and reach device
@@ -958,7 +960,8 @@ __device__ __forceinline__ int cache_slot(const TallyCache<nf> &L, uint32_t c) {
 }
 
 // 64-bit sums per slot of the transport's tally table, and words of a record
-// (Tallies::rec): the mixed gray engine tallies no path integral there.
+// (Tallies::rec): in the mixed gray engine the deposit and the path integral
+// share a word, one of them being 0 in every cell.
 template <typename Real, uint32_t F>
 struct TallyFields {
   static constexpr uint32_t nf = (sizeof(Real) == 4 && (F & kFeatMultigroup) == 0u) ? 1u : 2u;
@@ -1048,15 +1051,20 @@ struct DeviceSink {
     if (v != T(0)) atomicAdd(reinterpret_cast<T *>(rec) + static_cast<size_t>(c) * words + word, v);
   }
   // Whole values (below 2^62 quanta, as is every sum of them) into one word.
+  // With one sum (mixed gray engine) it takes both: a visit tallies a path
+  // integral only where nothing is absorbed.  (The path integral straight to
+  // its cell's word, all XCDs into one array, bounds such cells by that word:
+  // 4.6e8 segments of a 1000-cell slab that only scatters take 93.9 ms so, 10.8
+  // through the table and the records.)
   __device__ void visit(uint32_t c, fx::Limbs d, fx::Limbs e, uint32_t n) {
-    const unsigned long long dv = fx::value_of(d), ev = fx::value_of(e);
+    const unsigned long long ev = fx::value_of(e);
+    const unsigned long long dv = fx::value_of(d) + (nf < 2 ? ev : 0ull);
     const int s = cache_slot(cache, c);
     if (s >= 0) {
       if (dv) lds_add(&cache.at(0, s), dv);
       if (nf >= 2 && ev) lds_add(&cache.at(1, s), ev);
       lds_add(&cache.segs[s], n);
     }
-    if (nf < 2 && ev) atomicAdd(&args_at_use<Args>().t.pint[2 * c], ev);
     add_records<unsigned long long>(s < 0, c, dv, ev, n);
   }
   __device__ void roulette(uint32_t c, double w) { tally_limbs(args_at_use<Args>().t.rdep, c, fx::limbs_of(w, eq)); }
@@ -2129,7 +2137,8 @@ __global__ __launch_bounds__(256) void k_zero_ranges(ZeroRanges r) {
 
 // Sums the replicas of the per-visit tallies into dep, pint and segs, cell by
 // cell in replica order (integer sums are exact; the FP64 engine's sums are in
-// a fixed order); with 2-word records the transport has tallied pint itself.
+// a fixed order); the first of 2 words is dep where the cell absorbs
+// (`absorbs`: its sig_abs is positive) and pint elsewhere.
 // Also the check of the two-limb tallies' bound: a cell's low limbs take up
 // to 2^28 additions of values below 2^36 within 64 bits, so a cell with 2^28
 // or more segments in the step sets kErrTallyOverflow here, before the comb
@@ -2147,7 +2156,7 @@ __device__ __forceinline__ void fold_record(const Tallies &t, uint32_t c, T v[3]
   }
 }
 // Returns the cell's segments; `overflow`: more of them than its tallies hold.
-__device__ __forceinline__ uint32_t fold_cell(const Tallies &t, uint32_t c, bool &overflow) {
+__device__ __forceinline__ uint32_t fold_cell(const Tallies &t, uint32_t c, bool absorbs, bool &overflow) {
   uint64_t sg;
   if (t.dep_fp) {
     double v[3];
@@ -2158,19 +2167,22 @@ __device__ __forceinline__ uint32_t fold_cell(const Tallies &t, uint32_t c, bool
   } else {
     unsigned long long v[3];
     fold_record<unsigned long long>(t, c, v);
-    t.dep[2 * c] = v[0];
+    const bool path = t.rec_words == 2u && !absorbs;
+    t.dep[2 * c] = path ? 0ull : v[0];
     t.dep[2 * c + 1] = 0ull;
-    if (t.rec_words == 4u) t.pint[2 * c] = v[1];
+    t.pint[2 * c] = path ? v[0] : v[1];
     sg = v[2];
   }
   t.segs[c] = sg > 0xFFFFFFFFull ? 0xFFFFFFFFu : static_cast<uint32_t>(sg);
   overflow = sg >= (1ull << 28);
   return t.segs[c];
 }
-__global__ __launch_bounds__(256) void k_fold_replicas(Tallies t, uint32_t *__restrict__ err) {
+template <typename Real>
+__global__ __launch_bounds__(256) void k_fold_replicas(Tallies t, const CellXS<Real> *__restrict__ xs,
+                                                       uint32_t *__restrict__ err) {
   const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
   bool overflow = false;
-  if (c < t.ncell) fold_cell(t, c, overflow);
+  if (c < t.ncell) fold_cell(t, c, xs[c].sig_abs > Real(0), overflow);
   if (overflow) atomicOr(err, kErrTallyOverflow);
 }
 
@@ -2192,7 +2204,7 @@ __global__ __launch_bounds__(1024) void k_small_end(uint32_t N, PostArgs<Real> a
   bool overflow = (*a.err & kErrTallyOverflow) != 0u;
   for (uint32_t c = tid; c < N; c += 1024u) {
     bool o;
-    sg += fold_cell(a.t, c, o);
+    sg += fold_cell(a.t, c, a.xs[c].sig_abs > Real(0), o);
     overflow |= o;
   }
   for (int off = 32; off > 0; off >>= 1) sg += __shfl_xor(sg, off, 64);
