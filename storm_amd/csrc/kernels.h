@@ -999,6 +999,20 @@ __device__ __forceinline__ const Args &args_at_use() {
   return *(const Args *)p;
 }
 
+// The other way round, a pointer that every segment starts a chain of loads
+// from: the compiler read it again from the argument segment in each (FP64
+// pass kernel, 2 waves per SIMD: the 1-D slabs' step 1-2% slower for that
+// latency), and behind the asm it cannot.
+template <typename MeshT>
+__device__ __forceinline__ const MeshT &hold_width(const MeshT &m) {
+  return m;
+}
+__device__ __forceinline__ MeshView<double> hold_width(const MeshView<double> &m) {
+  MeshView<double> r = m;
+  asm volatile("" : "+s"(r.width));
+  return r;
+}
+
 template <typename Real, uint32_t F, typename MeshT>
 struct DeviceSink {
   using Args = TransportArgs<Real, MeshT>;
@@ -1152,6 +1166,7 @@ __device__ __forceinline__ void transport_chunks(const TransportArgs<Real, MeshT
   __syncthreads();
   DeviceSink<Real, F, MeshT> sink(a.k.eq, cache);
   const uint32_t chunks = a.chunks, n_in = a.n_in;
+  decltype(auto) mesh = hold_width(a.mesh);
   const uint32_t lane = __lane_id();
   const uint64_t base = static_cast<uint64_t>(blockIdx.x) * chunks * 64u;
   uint32_t escaped = 0, longest = 0;
@@ -1166,7 +1181,7 @@ __device__ __forceinline__ void transport_chunks(const TransportArgs<Real, MeshT
     Packet<Real> p;
     if (valid) {
       p = load_packet(args_at_use<Args>().in, static_cast<uint32_t>(i));
-      outcome = transport_packet<Real, F>(p, a.mesh, a.xs, a.acc, a.k, a.max_segments, sink);
+      outcome = transport_packet<Real, F>(p, mesh, a.xs, a.acc, a.k, a.max_segments, sink);
     }
     const bool alive = valid && outcome == kAlive;
     const bool census = valid && outcome == kCensus;
