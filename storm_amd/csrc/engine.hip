@@ -933,21 +933,6 @@ struct Engine final : EngineBase {
     return r;
   }
 
-  // Another schedule for the launches of one step, whatever ends it.
-  struct ScheduleHold {
-    LaunchPolicy &policy;
-    int32_t own = -1;
-    void set(int32_t s) {
-      own = policy.schedule;
-      policy.schedule = s;
-    }
-    void end() {
-      if (own >= 0) policy.schedule = own;
-      own = -1;
-    }
-    ~ScheduleHold() { end(); }
-  };
-
   // One transport launch on the kernel variant compiled for this problem's
   // features (random walk / DDMC, multigroup) and mesh, in the schedule in use.
   template <uint32_t F, typename MeshT>
@@ -1347,14 +1332,13 @@ struct Engine final : EngineBase {
     }
 
     // transport passes until every packet is in census, absorbed or gone
-    tune_before_step();
     // storm_gpu_step_noalloc, multigroup packets on polyhedral meshes: passes,
     // unless the launch was set or is being tuned.  Refill is faster there, but
     // its staged census takes 48 B a packet of the fixed scratch, which then
     // holds a fifth fewer packets of a step than it does with passes.
-    ScheduleHold hold{*this};
-    if (t_arena && watch && tune_phase < 0 && unstructured && groups >= 2 && precision != STORM_GPU_FP64)
-      hold.set(STORM_GPU_SCHEDULE_PASS);
+    const bool passes =
+        t_arena && watch && tune_phase < 0 && unstructured && groups >= 2 && precision != STORM_GPU_FP64;
+    StepLaunch step_launch(*this, passes ? STORM_GPU_SCHEDULE_PASS : -1);
     if (schedule == STORM_GPU_SCHEDULE_REFILL) cstage.ensure(n_total);
     counters.transport_block = block;
     counters.transport_chunks = chunks_per_wave();
@@ -1397,7 +1381,7 @@ struct Engine final : EngineBase {
       n_cen_total = h[1];
       ping = !ping;
     }
-    hold.end();
+    step_launch.restore();
     if (!small) k_fold_replicas<Real><<<blocks_for(N, 256), 256, 0, stream>>>(tal, xs.p, err.p);
     counters.seconds_transport = t_transport;
     counters.seconds_transport_max_launch = t_max;
@@ -1467,7 +1451,7 @@ struct Engine final : EngineBase {
     if (herr & kErrNegativeEnergy) throw EngineError(5, "Negative material internal energy in RadiationIMC");
     if (herr & kErrTallyOverflow)
       throw EngineError(5, "a cell received 2^28 tally additions in one step; the material state was not updated");
-    tune_after_step(static_cast<double>(counters.segments), counters.seconds_transport);
+    step_launch.done(static_cast<double>(counters.segments), counters.seconds_transport);
     auto t_end = std::chrono::steady_clock::now();
     counters.seconds_step = std::chrono::duration<double>(t_end - t_start).count();
   }

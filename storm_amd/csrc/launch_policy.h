@@ -80,7 +80,8 @@ struct LaunchPolicy {
   // cold start that the random walk dominates, a heated region that then
   // spreads), and so may the faster schedule (refill leads on the large
   // problems measured, 6.1 against 11.5 ms a step on the 64^3 cube; on the
-  // 100-cell slab of 1e5 packets pass is about 10% faster).  Every watch_every steps one step runs in the other
+  // 100-cell slab of 1e5 packets pass is about 10% faster).  Every
+  // watch_every steps one step runs in the other
   // schedule; its rate is compared with the mean of the steps either side of
   // it (which cancels a steady trend) and the engine switches when the other
   // is more than 3% faster.  A probe that loses by more than 10% doubles the
@@ -102,6 +103,15 @@ struct LaunchPolicy {
   }
   static int32_t other(int32_t s) {
     return s == STORM_GPU_SCHEDULE_REFILL ? STORM_GPU_SCHEDULE_PASS : STORM_GPU_SCHEDULE_REFILL;
+  }
+
+  // A step that the engine runs in a schedule of its own choice says nothing
+  // about the schedules the watch compares, and the steps either side of it are
+  // not next to each other: a probe that it would fall into is dropped.
+  void watch_drop_probe() {
+    if (watch_state == 1) schedule = other(schedule);
+    if (watch_state != 0) watch_n = 0;
+    watch_state = 0;
   }
 
   void tune_before_step() {
@@ -154,6 +164,33 @@ struct LaunchPolicy {
       watch_n = 0;
     }
   }
+};
+
+// One step's launches: in the policy's schedule, whose rate the policy then
+// learns, or in the schedule `set` (not -1), which leaves the policy as it was.
+struct StepLaunch {
+  LaunchPolicy &policy;
+  const bool held;
+  int32_t own = -1;
+  StepLaunch(LaunchPolicy &p, int32_t set) : policy(p), held(set >= 0) {
+    if (!held) {
+      policy.tune_before_step();
+      return;
+    }
+    policy.watch_drop_probe();
+    own = policy.schedule;
+    policy.schedule = set;
+  }
+  // the transport is over (or the step, however it ends)
+  void restore() {
+    if (own >= 0) policy.schedule = own;
+    own = -1;
+  }
+  void done(double segments, double seconds) {
+    restore();
+    if (!held) policy.tune_after_step(segments, seconds);
+  }
+  ~StepLaunch() { restore(); }
 };
 
 }  // namespace gpu

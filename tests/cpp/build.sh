@@ -19,3 +19,6 @@ mv "$here/_build/manager_groups.tmp" "$here/_build/manager_groups"
 g++ -std=c++17 -O2 -Wall -Wextra -I"$root/include" -I"$root/storm_amd/csrc" -o "$here/_build/launch_policy.tmp" \
   "$here/launch_policy.cpp"
 mv "$here/_build/launch_policy.tmp" "$here/_build/launch_policy"
+g++ -std=c++17 -O2 -Wall -Wextra -I"$root/include" -I"$root/storm_amd/csrc" -o "$here/_build/launch_hold.tmp" \
+  "$here/launch_hold.cpp"
+mv "$here/_build/launch_hold.tmp" "$here/_build/launch_hold"
