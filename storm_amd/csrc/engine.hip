@@ -1043,6 +1043,24 @@ struct Engine final : EngineBase {
     }
   };
 
+  // The per-visit tallies of a step whose transport has started, summed over
+  // the replicas once: by now(), by k_small_end, or where the step stops in
+  // between, so that the segment counts and tallies read after it are its own
+  // (after status 6 they show the cells where histories are stuck).
+  struct FoldPending {
+    Engine &e;
+    bool pending = true;
+    void now() {
+      pending = false;
+      k_fold_replicas<Real><<<blocks_for(e.N, 256), 256, 0, e.stream>>>(e.tal, e.xs.p, e.err.p);
+    }
+    ~FoldPending() {
+      if (!pending) return;
+      now();
+      (void)hipStreamSynchronize(e.stream);
+    }
+  };
+
   bool failed_ = false;  // a step stopped part-way with status 5
   void step(double dt) override {
     if (failed_)
@@ -1061,7 +1079,7 @@ struct Engine final : EngineBase {
       ZeroBatch z;
       zero_add(z, tally_u64.p, tally_u64.n * sizeof(unsigned long long));
       if (precision == STORM_GPU_FP64) zero_add(z, tally_f64.p, tally_f64.n * sizeof(double));
-      zero_add(z, tal.begin, static_cast<size_t>(N) * sizeof(uint32_t));
+      zero_add(z, segs_begin_->p, 2 * static_cast<size_t>(N) * sizeof(uint32_t));
       zero_add(z, tal.eg, static_cast<size_t>(N) * tal.eg_groups * sizeof(unsigned long long));
       zero_add(z, tal.eg_fp, static_cast<size_t>(N) * tal.eg_groups * sizeof(double));
       zero_add(z, rec.p, static_cast<size_t>(kTallyReplicas) * N * tal.rec_words * sizeof(unsigned long long));
@@ -1345,6 +1363,7 @@ struct Engine final : EngineBase {
     counters.transport_schedule = schedule;
     const MeshView<Real> mv = meshview();
     const AccelView<Real> av = accelview();
+    FoldPending fold{*this};
     uint64_t n_in = n_total;
     bool ping = true;
     double t_transport = 0.0, t_max = 0.0;
@@ -1382,7 +1401,7 @@ struct Engine final : EngineBase {
       ping = !ping;
     }
     step_launch.restore();
-    if (!small) k_fold_replicas<Real><<<blocks_for(N, 256), 256, 0, stream>>>(tal, xs.p, err.p);
+    if (!small) fold.now();  // a small problem's are folded by k_small_end
     counters.seconds_transport = t_transport;
     counters.seconds_transport_max_launch = t_max;
     counters.census_before_comb = n_cen_total;
@@ -1420,6 +1439,7 @@ struct Engine final : EngineBase {
     const unsigned long long *hp = mail_h;
     if (small) {
       k_small_end<Real><<<1, 1024, 0, stream>>>(N, post, dsc.p, leaving.p, mail_h);
+      fold.pending = false;
       HIPCHECK(hipStreamSynchronize(stream));
     } else {
       k_post<Real><<<blocks_for(N, 256), 256, 0, stream>>>(N, post);

@@ -2156,9 +2156,10 @@ __global__ __launch_bounds__(256) void k_zero_ranges(ZeroRanges r) {
 // (`absorbs`: its sig_abs is positive) and pint elsewhere.
 // Also the check of the two-limb tallies' bound: a cell's low limbs take up
 // to 2^28 additions of values below 2^36 within 64 bits, so a cell with 2^28
-// or more segments in the step sets kErrTallyOverflow here, before the comb
-// and postStep, and postStep then commits nothing.  The segment count
-// saturates at 2^32 - 1.
+// or more segments in the step sets kErrTallyOverflow here, before postStep,
+// which then commits nothing (the comb, which runs before this in a small
+// problem's step and after it in others, does not look at these tallies).
+// The segment count saturates at 2^32 - 1.
 template <typename T>
 __device__ __forceinline__ void fold_record(const Tallies &t, uint32_t c, T v[3]) {
   const T *rec = reinterpret_cast<const T *>(t.rec);
