@@ -1205,11 +1205,15 @@ __device__ __forceinline__ void transport_chunks(const TransportArgs<Real, MeshT
 }
 
 // Waves per SIMD the pass kernel is compiled for: in FP32 the most that leave
-// it without spills (80-96 VGPRs at 5, up to 124 at 4).  A spill is more than
-// its traffic: this compiler stores some before the wavefront's lanes are all
-// switched on again at the end of a branch, and a value that the other lanes
-// still need is then lost (seen in the escape and walk counters of a build
-// that spilled 100 bytes).  FP64: the compiler's choice (2-3 waves).
+// it without spills (90 and 94 VGPRs at 5, 103-123 at 4); FP64: the compiler's
+// choice (2-3 waves).  No transport kernel spills a vector register, and
+// check_registers.py fails a build that does: an earlier form that spilled 100
+// bytes counted escapes and walk steps wrongly.  These are what a wavefront's
+// idle lanes hold while others run, so a spill stored while only some lanes
+// are on would explain it, but that was not shown: that build was not kept,
+// and the present code compiled for 6, 7 and 8 waves (10 to 74 spills and
+// reloads a kernel) has none ahead of a branch's end, where the lanes are
+// switched on again.
 template <typename Real, uint32_t F, typename MeshT>
 struct TransportWaves {
   static constexpr int kMin = sizeof(Real) == 8 ? 1 : (F ? 4 : 5);
