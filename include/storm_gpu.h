@@ -299,7 +299,8 @@ int storm_gpu_debug_spectrum(storm_gpu_engine *eng, int32_t *groups, double *nu_
  * `count` floats whose bit patterns start at `first`, how many differ from
  * the IEEE operation or the full function they stand for (op 0 reciprocal,
  * 1 square root, 2 logarithm of a uniform, 3 e^x - 1 for x <= 0, 4 quotients
- * of pairs made from the patterns).  No counterpart in the reference. */
+ * of pairs made from the patterns, 5 the median of such a pair and no number).
+ * No counterpart in the reference. */
 int storm_gpu_debug_math(int32_t op, uint32_t first, uint64_t count, uint64_t *mismatches);
 
 /* Measurement aid with no counterpart in the reference: one plain copy of

@@ -20,8 +20,10 @@
 //           and cos on [-pi/4, pi/4].
 //   1/x, sqrt, a/b (recip_f, sqrt_f, div_f): the hardware's 1 ulp estimate
 //           and one Newton step with a fused remainder, which rounds as IEEE
-//           does over the ranges stated at each (checked for every float of
-//           the range on gfx950); the host uses the IEEE operators.
+//           does over the ranges stated at each (on gfx950 1/x and sqrt are
+//           checked for every float of the range; a/b, whose rounding follows
+//           from the theorem named there, for 2^28 pairs); the host uses the
+//           IEEE operators.
 // Accuracy is a few ulp, far below Monte Carlo noise; what matters is that
 // host and device produce the same bits.
 #pragma once
@@ -87,8 +89,8 @@ STORM_HD float sqrt_f(float x) {
 #endif
 }
 
-// a / b as IEEE rounds it, for b within [2^-60, 2^60] and a 0 or within
-// [2^-60, 2^60] (signs free): with the correctly rounded reciprocal the
+// a / b as IEEE rounds it, for |b| within [2^-60, 2^60] and a +0 or |a| within
+// [2^-60, 2^60]: with the correctly rounded reciprocal the
 // quotient corrected by its exact remainder is correctly rounded (Markstein
 // 1990).
 STORM_HD float div_f(float a, float b) {

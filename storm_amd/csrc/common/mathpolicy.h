@@ -25,7 +25,7 @@ struct MathPolicy<float> {
   STORM_HD static float recip_any(float x) {
     return (x >= 0x1p-126f && x <= 0x1p126f) ? fpm::recip_f(x) : 1.0f / x;
   }
-  // a / b, rounded as IEEE does for b within [2^-60, 2^60] and a 0 or within
+  // a / b, rounded as IEEE does for b within [2^-60, 2^60] and a +0 or within
   // [2^-60, 2^60]; elsewhere about it, or no number
   STORM_HD static float div_tame(float a, float b) { return fpm::div_f(a, b); }
   // the middle one of three, the smaller of the others if one is no number

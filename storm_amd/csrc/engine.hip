@@ -2140,15 +2140,18 @@ int storm_gpu_device_info(char *buf, size_t len) {
 
 int storm_gpu_debug_math(int32_t op, uint32_t first, uint64_t count, uint64_t *mismatches) {
   return guarded([&] {
-    if (op < 0 || op > 4 || !mismatches) throw EngineError(1, "op must be 0 .. 4 and mismatches given");
+    if (op < 0 || op > 5 || !mismatches) throw EngineError(1, "op must be 0 .. 5 and mismatches given");
     if (count > (1ull << 32)) throw EngineError(1, "at most 2^32 bit patterns");
     DevBuf<unsigned long long> bad;
-    bad.ensure(1);
-    k_fill_u64<<<1, 64>>>(bad.p, 1, 0ull);
+    bad.ensure(2);
+    k_fill_u64<<<1, 64>>>(bad.p, 2, 0ull);
+    HIPCHECK(hipGetLastError());
     if (count) k_check_math<<<4096, 256>>>(op, first, count, bad.p);
-    unsigned long long h = 0;
-    HIPCHECK(hipMemcpy(&h, bad.p, sizeof h, hipMemcpyDeviceToHost));
-    *mismatches = h;
+    HIPCHECK(hipGetLastError());
+    unsigned long long h[2] = {0, 0};
+    HIPCHECK(hipMemcpy(h, bad.p, sizeof h, hipMemcpyDeviceToHost));
+    if (h[1] != count) throw EngineError(2, "the check did not look at every pattern");
+    *mismatches = h[0];
   });
 }
 

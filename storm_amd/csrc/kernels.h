@@ -2251,11 +2251,13 @@ __global__ __launch_bounds__(1024) void k_small_end(uint32_t N, PostArgs<Real> a
 // Counts the floats among the n bit patterns from `first` on where a short
 // form of fpmath.h differs from what it stands for: 0 recip_f and 1 / x,
 // 1 sqrt_f and sqrtf, 2 log_unit and logf_d, 3 expm1_neg and expm1f_d, 4 div_f
-// and a / b for a pair made from each pattern with exponents within 2^-60 ..
-// 2^60.
+// and a / b for a pair made from each pattern, b's exponent and a's within
+// 2^-60 .. 2^60 (one in 20 at either end) and a +0 in one of 64, 5 median of a
+// pair and no number, and the smaller of the pair.  bad[0]: patterns that
+// differ, bad[1]: patterns looked at.
 __global__ __launch_bounds__(256) void k_check_math(int32_t op, uint32_t first, uint64_t n,
                                                     unsigned long long *__restrict__ bad) {
-  uint32_t wrong = 0u;
+  uint32_t wrong = 0u, seen = 0u;
   for (uint64_t i = blockIdx.x * 256ull + threadIdx.x; i < n; i += gridDim.x * 256ull) {
     const uint32_t b = first + static_cast<uint32_t>(i);
     const float x = fpm::u2f(b);
@@ -2275,16 +2277,30 @@ __global__ __launch_bounds__(256) void k_check_math(int32_t op, uint32_t first, 
     } else {
       const Philox4 r = philox4x32_10(b, 0u, 0u, 0u, 1u, 2u);
       auto within = [](uint32_t w, uint32_t e) {
-        return fpm::u2f((w & 0x807FFFFFu) | ((67u + e % 121u) << 23));  // 2^-60 .. 2^60
+        e %= 128u;
+        e = e < 121u ? e : (e & 1u ? 0u : 120u);
+        return fpm::u2f((w & 0x807FFFFFu) | ((67u + e) << 23));  // 2^-60 .. 2^60
       };
-      const float p = within(r.v[0], r.v[2]), q = within(r.v[1], r.v[3]);
-      got = fpm::div_f(p, q);
-      want = p / q;
+      const float p = (b & 63u) ? within(r.v[0], r.v[2]) : 0.0f, q = within(r.v[1], r.v[3]);
+      if (op == 4) {
+        got = fpm::div_f(p, q);
+        want = p / q;
+      } else {
+        got = MathPolicy<float>::median(p, q, fpm::u2f(0x7FC00000u));
+        want = p < q ? p : q;
+      }
     }
     wrong += fpm::f2u(got) != fpm::f2u(want) ? 1u : 0u;
+    ++seen;
   }
-  for (int off = 32; off > 0; off >>= 1) wrong += __shfl_xor(wrong, off, 64);
-  if (wrong && __lane_id() == 0u) atomicAdd(bad, static_cast<unsigned long long>(wrong));
+  for (int off = 32; off > 0; off >>= 1) {
+    wrong += __shfl_xor(wrong, off, 64);
+    seen += __shfl_xor(seen, off, 64);
+  }
+  if (__lane_id() == 0u) {
+    if (wrong) atomicAdd(bad, static_cast<unsigned long long>(wrong));
+    if (seen) atomicAdd(bad + 1, static_cast<unsigned long long>(seen));
+  }
 }
 
 // Plain copy of n 16-byte words, one per thread: a kernel whose HBM traffic
