@@ -295,6 +295,12 @@ int storm_gpu_debug_accel(storm_gpu_engine *eng, void *out, uint64_t *bytes);
 int storm_gpu_debug_spectrum(storm_gpu_engine *eng, int32_t *groups, double *nu_pow, void *bounds_kev, void *cdf,
                              void *sig_s);
 
+/* Whether steps of a small problem (up to 2048 cells) start and end with the
+ * launches of larger ones instead of one block each (0, the default: one
+ * block each), for comparing the two; results do not depend on it.  No
+ * counterpart in the reference. */
+int storm_gpu_debug_general_steps(storm_gpu_engine *eng, int32_t enable);
+
 /* Checks the mixed engine's short arithmetic forms on the device: over the
  * `count` floats whose bit patterns start at `first`, how many differ from
  * the IEEE operation or the full function they stand for (op 0 reciprocal,

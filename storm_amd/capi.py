@@ -169,6 +169,7 @@ def load_library(path: str | None = None):
                                      C.POINTER(C.c_uint64), C.POINTER(C.c_uint32)], C.c_int),
         "storm_gpu_debug_accel": ([vp, vp, C.POINTER(C.c_uint64)], C.c_int),
         "storm_gpu_debug_spectrum": ([vp, C.POINTER(C.c_int32), C.POINTER(C.c_double), vp, vp, vp], C.c_int),
+        "storm_gpu_debug_general_steps": ([vp, C.c_int32], C.c_int),
         "storm_gpu_debug_math": ([C.c_int32, C.c_uint32, C.c_uint64, C.POINTER(C.c_uint64)], C.c_int),
         "storm_gpu_calibration_copy": ([C.c_uint64, C.POINTER(C.c_double)], C.c_int),
         "storm_voronoi_build": ([_dp, C.c_uint32, _dp, _dp, C.POINTER(vp)], C.c_int),

@@ -237,6 +237,7 @@ struct EngineBase : LaunchPolicy {
   double source_T = 0.0;
   int32_t seg_per_pass = 1 << 20;
   bool keep_inputs = false;
+  bool general_steps = false;
 };
 
 template <typename Real>
@@ -1091,7 +1092,7 @@ struct Engine final : EngineBase {
     }
     eq_prev_ledger_ = eq_prev;
     const uint32_t M = 1u << morton.total;
-    const bool small = inst.empty() && N <= kSmallCells && M <= kSmallCodes;
+    const bool small = !general_steps && inst.empty() && N <= kSmallCells && M <= kSmallCodes;
     if (!small) sum_async(e_mat.p, N, dsc.p);  // material energy before the step, read by the ledger
     if (!inst.empty())
       k_inst_sum<<<static_cast<uint32_t>(inst.size()), 256, 0, stream>>>(d_inst_first.p, e_mat.p, d_inst_mat0.p);
@@ -2311,6 +2312,10 @@ int storm_gpu_get_launch(storm_gpu_engine *eng, int32_t *block_size, int32_t *ch
     *schedule = e->schedule;
     *tuning = e->tune_phase >= 0 ? 1 : 0;
   });
+}
+
+int storm_gpu_debug_general_steps(storm_gpu_engine *eng, int32_t enable) {
+  return guarded([&] { as_engine(eng)->general_steps = enable != 0; });
 }
 
 int storm_gpu_debug_keep_transport_inputs(storm_gpu_engine *eng, int32_t enable) {

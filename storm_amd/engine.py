@@ -164,6 +164,10 @@ class GpuEngine:
         ptr = recs.ctypes.data_as(C.POINTER(capi.PacketRecord))
         self._check(self.lib.storm_gpu_import_census(self.h, ptr, n))
 
+    def general_steps(self, enable: bool = True):
+        """Steps of a small problem run the launches of larger ones (storm_gpu_debug_general_steps)."""
+        self._check(self.lib.storm_gpu_debug_general_steps(self.h, 1 if enable else 0))
+
     # -- replay support
     def keep_transport_inputs(self, enable: bool = True):
         self._check(self.lib.storm_gpu_debug_keep_transport_inputs(self.h, 1 if enable else 0))
