@@ -325,8 +325,9 @@ def c5_line(W, K, log):
     per = dict(segments=0, wall=0.0, transport=0.0, packets=0, rw=0, ddmc=0)
     t0 = time.perf_counter()
     for i, d in enumerate(inst):
-        # the pass schedule: faster than the FP64 engine's default lane
-        # refill on these small slabs (16.0 against 14.8 G segments/s)
+        # the pass schedule, as this line has always run them (the FP64
+        # engine's default lane refill is 1-2% faster on these small slabs:
+        # 18.7 against 18.4 G segments/s)
         r = _run_steps(P.c5_instance_spec(d, seed=1 + i, steps=W + K), capi.FP64, W + K, W, None, "",
                        schedule=capi.SCHEDULE_PASS)
         for k in per:

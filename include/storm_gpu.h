@@ -231,18 +231,20 @@ int storm_gpu_queue_source_packets(storm_gpu_engine *eng, const storm_packet_rec
  * wavefront (storm_gpu_set_chunks_per_wave; each schedule keeps its own,
  * 2 for PASS and 8 for REFILL by default, 16 for REFILL in the FP64 engine;
  * in the mixed engine on polyhedral meshes 4 for REFILL, and 1 for PASS on
- * multigroup problems; 16 for REFILL, in 512-thread blocks, on Cartesian
- * problems with DDMC; blocks are otherwise 256 threads; a launch takes 8 for
- * 16 when it would be less than two and a half rounds of the blocks that the
- * device holds at once, and halves it while it would be less than one).  The
- * engine starts in REFILL (storm_gpu_step_noalloc runs multigroup polyhedral
- * problems of the mixed engine in PASS, which needs less scratch, unless the
- * launch was set or is being tuned) and watches: after 16 steps one
- * step runs in the other schedule, and the engine switches when that one
- * moved more transport segments per second than the mean of the steps
- * either side of it, by more than 3%; the next probe follows 16 steps later,
- * or twice the last interval (at most 128) when the probe lost by more than
- * 10%.  A block size other than 0 fixes the launch and stops the watch.  A packet's history does not depend on the schedule, the block
+ * multigroup problems; 16 for REFILL, in 512-thread blocks, in the mixed
+ * engine on Cartesian problems with DDMC; blocks are otherwise 256 threads;
+ * a launch takes 8 for 16 when it would be less than two and a half rounds of
+ * the blocks that the device holds at once, and halves it while it would be
+ * less than one).  The engine starts in REFILL (storm_gpu_step_noalloc runs
+ * multigroup polyhedral problems of the mixed engine in PASS, which needs less
+ * scratch, unless the launch was set or is being tuned; the watch takes no
+ * notice of such steps) and watches: after 16 steps one step runs in the other
+ * schedule, and the engine switches when that one moved more transport segments
+ * per second than the mean of the steps either side of it, by more than 3%; the
+ * next probe follows 16 steps later, or twice the last interval (at most 128)
+ * when the probe lost by more than 10%.  A block size other than 0 fixes the
+ * launch and stops the watch.  A packet's history does not depend on the
+ * schedule, the block
  * size or the chunks per wavefront, only on segments_per_pass: the mixed
  * engine's results are bit-identical across them, the FP64 engine's tallies
  * differ only in the order of their floating-point sums.  With block size 0

@@ -444,19 +444,22 @@ struct Engine final : EngineBase {
     // The starting launch (the watch corrects the schedule as the problem
     // evolves), measured in ms of transport per step: lanes refill, from ranges
     // of 8 chunks per wavefront in 256-thread blocks (the 64^3 cube over 45
-    // steps: 6.1 against 6.7 from 4 and 8.0 from 16, whose cells no longer fit
-    // the LDS table; passes 11.5), of 4 in the mixed engine on polyhedral
-    // meshes (32 slabs in a batch 5.9 against 6.5 from 8; 64 groups on 3e4
-    // cells 4.9 against 4.9, passes 5.8).
+    // steps: 5.6 against 5.8 from 4 and 7.4 from 16, whose cells no longer fit
+    // the LDS table; passes 9.6), of 4 in the mixed engine on polyhedral
+    // meshes (32 slabs in a batch 5.7 against 6.5 from 8; 64 groups on 3e4
+    // cells 7.7 against 7.5, passes 10.7).
     schedule = STORM_GPU_SCHEDULE_REFILL;
     if (unstructured && precision != STORM_GPU_FP64) chunks_of[1] = 4;
     if (unstructured && precision != STORM_GPU_FP64 && p->groups.num_groups >= 2) chunks_of[0] = 1;
     // the FP64 engine from 16 (its 2-3 waves per SIMD leave each block a larger
-    // LDS table): the 64^3 cube 13.2 against 13.9 from 8
+    // LDS table): the 64^3 cube 11.3 against 11.9 from 8 (10.6 from 16 in
+    // 128-thread blocks), though the step slab 15.1 against 14.5
     if (precision == STORM_GPU_FP64) chunks_of[1] = 16;
-    // the mixed engine with DDMC on a Cartesian mesh from 16 in 512-thread
-    // blocks (the step slab over 45 steps: 11.8, in 256-thread blocks of 8 12.4;
-    // a launch of few rounds takes 8, launch_chunks)
+    // the mixed engine with DDMC on a Cartesian mesh in 512-thread blocks (the
+    // step slab over 45 steps 11.4 from 16, 10.8 from 8; in 256-thread blocks
+    // 14.1 and 12.3).  16 is no longer the better range: 8 leads on 200x12x12
+    // cells too, 5.2 against 5.8.  (A launch of few rounds takes 8,
+    // launch_chunks.)
     if (!unstructured && imc.with_ddmc && precision != STORM_GPU_FP64) {
       block = 512;
       chunks_of[1] = 16;

@@ -1211,9 +1211,9 @@ __device__ __forceinline__ void transport_chunks(const TransportArgs<Real, MeshT
 // bytes counted escapes and walk steps wrongly.  These are what a wavefront's
 // idle lanes hold while others run, so a spill stored while only some lanes
 // are on would explain it, but that was not shown: that build was not kept,
-// and the present code compiled for 6, 7 and 8 waves (10 to 74 spills and
-// reloads a kernel) has none ahead of a branch's end, where the lanes are
-// switched on again.
+// and the present code compiled for 6, 7 and 8 waves (three kernels, 10 to 74
+// spills and reloads each) has none ahead of a branch's end, where the lanes
+// are switched on again.
 template <typename Real, uint32_t F, typename MeshT>
 struct TransportWaves {
   static constexpr int kMin = sizeof(Real) == 8 ? 1 : (F ? 4 : 5);

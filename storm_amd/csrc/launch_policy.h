@@ -79,12 +79,11 @@ struct LaunchPolicy {
   // The schedule watch.  The workload of a problem changes as it runs (a
   // cold start that the random walk dominates, a heated region that then
   // spreads), and so may the faster schedule (refill leads on the large
-  // problems measured, 6.1 against 11.5 ms a step on the 64^3 cube; on the
-  // 100-cell slab of 1e5 packets pass is about 10% faster).  Every
-  // watch_every steps one step runs in the other
-  // schedule; its rate is compared with the mean of the steps either side of
-  // it (which cancels a steady trend) and the engine switches when the other
-  // is more than 3% faster.  A probe that loses by more than 10% doubles the
+  // problems measured, 5.6 against 9.6 ms a step on the 64^3 cube; on the
+  // 100-cell slab of 1e5 packets pass is 3% faster).  Every watch_every steps
+  // one step runs in the other schedule; its rate is compared with the mean of
+  // the steps either side of it (which cancels a steady trend) and the engine
+  // switches when the other is more than 3% faster.  A probe that loses by more than 10% doubles the
   // interval (16 steps at first, at most 128), a switch resets it: a problem
   // runs hundreds to thousands of steps and its workload drifts over tens,
   // while each probe of a clearly slower schedule costs its margin.  On
