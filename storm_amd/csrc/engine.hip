@@ -932,7 +932,7 @@ struct Engine final : EngineBase {
   uint32_t groups_of(KernelFit &f, int32_t ch, uint32_t nf) {
     uint32_t &r = f.groups[chunk_index(ch)];
     if (!r)
-      r = cache_groups(static_cast<uint32_t>(block) * static_cast<uint32_t>(ch), nf, f.per_cu,
+      r = cache_groups(static_cast<uint32_t>(block) * static_cast<uint32_t>(ch), N, nf, f.per_cu,
                        static_cast<uint32_t>(block) / 64u);
     return r;
   }

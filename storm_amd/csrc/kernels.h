@@ -886,10 +886,16 @@ constexpr uint32_t kCacheProbes = 2;
 inline __host__ __device__ uint32_t cache_bytes(uint32_t groups, uint32_t nf, uint32_t waves) {
   return waves * 64u * 8u * (nf + 1u) + 4u * groups * (8u * nf + 8u) + 16u;
 }
-// Most groups within one group per packet of the block's range and the LDS
-// share of one block when `blocks_per_cu` blocks are resident (LDS is handed
-// out in pieces of 1280 bytes).
-inline uint32_t cache_groups(uint32_t packets, uint32_t nf, uint32_t blocks_per_cu, uint32_t waves) {
+// Most groups within the LDS share of one block when `blocks_per_cu` blocks are
+// resident (LDS is handed out in pieces of 1280 bytes) and one group per packet
+// of the block's range, or as many as hold all of the mesh's `cells` twice
+// where these are more: few packets cross many cells when they are thin, and a
+// visit that finds no slot costs its wavefront the whole of add_records (2000
+// cells, 3e4 packets, ranges of 256: 256 groups 1.80 ms in FP64 and 1.51 mixed,
+// this many 1.43 and 1.33, a table that holds the cells once 1.46 and 1.33; 3000
+// cells 2.88 and 2.53, 2.18 and 2.16).
+inline uint32_t cache_groups(uint32_t range, uint32_t cells, uint32_t nf, uint32_t blocks_per_cu, uint32_t waves) {
+  const uint32_t all = (cells + 1u) / 2u, packets = range < all ? all : range;
   const uint32_t share = (160u * 1024u) / (blocks_per_cu ? blocks_per_cu : 1u) / 1280u * 1280u;
   const uint32_t fixed = cache_bytes(0u, nf, waves);
   const uint32_t room = share > fixed ? (share - fixed) / (4u * (8u * nf + 8u)) : 1u;
@@ -1009,7 +1015,7 @@ __device__ __forceinline__ const MeshT &hold_width(const MeshT &m) {
 }
 __device__ __forceinline__ MeshView<double> hold_width(const MeshView<double> &m) {
   MeshView<double> r = m;
-  asm volatile("" : "+s"(r.width));
+  asm volatile("" : "+s"(r.width));  // (its loads become flat ones: 1% better than global ones here)
   return r;
 }
 
